@@ -19,7 +19,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libjanis_hip.so")
-SOURCES = ["runtime.hip", "qmv.hip", "qmm.hip", "gather.hip", "dequant.hip", "decode.hip", "ops.hip"]
+SOURCES = ["runtime.hip", "qmv.hip", "qmm.hip", "gather.hip", "dequant.hip", "decode.hip", "attention.hip", "ops.hip"]
 # bench.py's measurement kernels (plain read, copy): a library of their own,
 # outside the backend's C ABI
 BENCH_SOURCE = "bench_kernels.hip"

@@ -1,0 +1,459 @@
+// SDPA with several query rows per head (prompts; cpu/cpu_attn.go:64-119) on
+// the matrix cores of gfx950: head_dim 128, bf16 or f16 keys and values, bf16
+// or fp32 queries, any Hq / Hk, the offset causal mask.
+//
+// A block of 4 waves takes 128 rows of one kv head -- row r is query r / G of
+// head r % G, so the heads that share the keys read them from LDS once -- and
+// walks the keys in tiles of 64 with an online softmax; a wave owns 32 rows.
+// Both products run transposed, S^T = K Q^T and O^T = V^T P^T, so that a lane
+// holds one row (lane % 32) in both accumulators: the row's maximum, sum and
+// rescale are per-lane scalars, and the scores become the second product's B
+// operand where they are, with no exchange between lanes (its K order is the
+// order the first product left the keys in, applied to V as it is staged).
+//
+// Precision is that of fp32 arithmetic. Keys and values enter as they are
+// stored. Queries and probabilities are fp32 and enter as sums of 16-bit terms,
+// one matrix instruction per term into the same fp32 accumulator:
+//   f16 keys:  a row of q times a power of two that brings its largest element
+//              to [2^13, 2^14) (its inverse joins the softmax scale), as one f16
+//              term for bf16 q (exact) and two for fp32 q (22 bits and a sign);
+//              p * 2^7 as two f16 terms;
+//   bf16 keys: one bf16 term for bf16 q, three for fp32 q (24 bits); p as three
+//              bf16 terms.
+// Relative error against float64 with scores of standard deviation 2.3, 512 and
+// 4000 keys: 3.9e-7 and 7.9e-7 (fp32 q, f16 keys), where the per-row kernel
+// (sdpa_rows_kernel) has 7.3e-7 and 1.5e-6; with bf16 q and keys 2.8e-7 and
+// 6.9e-7 against 3.8e-7 and 1.1e-6.
+//
+// The products also meet keys past a row's limit with p = 0, where an infinity
+// or NaN in V would give NaN; the per-row kernel never reads those. So a row
+// whose result is not finite is computed again the way that kernel does (same
+// operations in the same order over the block's keys), and that result stands.
+//
+// Bound: the matrix cores, with the softmax's VALU work beside them: per 32
+// rows x 64 keys, 16 MFMAs for each q term and 16 for each p term (512 cycles
+// each 16) against ~1100 cycles of VALU. K/V tiles come through registers into
+// two LDS buffers (64 KiB: two blocks per CU), the next tile's loads in flight
+// during the current one. Measured on MI355X, 32 heads over 8 (calls from the
+// host, the per-row kernel before): 512 queries of 512 keys 3433 -> 46 us (fp32
+// q, f16 keys), 1500 of 4000 144.9 ms -> 222 us (bf16), 16 of 4112 2.9 ms -> 37 us.
+#include "jh_common.hpp"
+
+namespace jh {
+namespace {
+
+constexpr int kDh = 128;
+constexpr int kRows = 128;  // rows per block
+constexpr int kKeys = 64;   // keys per tile
+constexpr int kTileBytes = kKeys * kDh * 2;
+constexpr float kLog2e = 1.44269504088896340736f;
+constexpr float kPShift = 7.0f;   // p is held as p * 2^7
+constexpr float kLazy = 8.0f;     // a row's maximum is moved when it grew by more than this (log2)
+
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ float load_act(const void* p, int64_t i, int dt) {
+    return dt == JH_BF16 ? bf16_to_f32(static_cast<const uint16_t*>(p)[i]) : static_cast<const float*>(p)[i];
+}
+
+template <bool F16>
+__device__ __forceinline__ floatx16 mfma(uint4 a, uint4 b, floatx16 c) {
+    if constexpr (F16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c,
+                                                      0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
+                                                       c, 0, 0, 0);
+}
+
+// (a, b) as N packed 16-bit terms, each the nearest to what the earlier ones
+// left (the remainders are exact in fp32).
+template <bool F16, int N>
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t (&t)[N]) {
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+        const f32x2_t f = {a, b};
+        if constexpr (F16) {
+            const f16x2_t v = __builtin_convertvector(f, f16x2_t);
+            t[n] = __builtin_bit_cast(uint32_t, v);
+            a -= (float)v.x;
+            b -= (float)v.y;
+        } else {
+            t[n] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
+            a -= __uint_as_float(t[n] << 16);
+            b -= __uint_as_float(t[n] & 0xFFFF0000u);
+        }
+    }
+}
+
+__device__ __forceinline__ bool finite(float v) { return (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u; }
+
+struct SdpaArgs {
+    const void* q;
+    int q_dt;
+    const uint16_t *k, *v;
+    void* out;
+    int out_dt;
+    int Hk, G, Lq, Lk, n_tiles, BHk;
+    int64_t kcap;
+    float scale;
+    int causal;
+    int kps;      // keys per split (a multiple of kKeys)
+    int nsplit;
+    float* part_o;   // [B*Hk * G*Lq, nsplit, 128] (split)
+    float* part_ml;  // [B*Hk * G*Lq, nsplit, 2]
+};
+
+// F16: f16 keys and values (else bf16). QN: 16-bit terms of q.
+template <bool F16, int QN, bool SPLIT>
+__global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArgs a) {
+    constexpr int PN = F16 ? 2 : 3;
+    // two slots of a key tile [64][128] (16-byte chunk c of key k at c ^ (k % 16))
+    // and a value tile transposed, [128][64] (4-key chunk s of feature d at
+    // s ^ (d / 2 % 16)): every fragment read below spreads over all banks
+    __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kTileBytes];
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // heads fastest: with 8 kv heads a head's tiles share one XCD's L2; tiles
+    // from the last (the longest under the causal mask)
+    const int bhk = blockIdx.x % a.BHk, tile = a.n_tiles - 1 - blockIdx.x / a.BHk;
+    const int b = bhk / a.Hk, hk = bhk - b * a.Hk;
+    const int n_rows = a.G * a.Lq;
+    auto limit_of = [&](int r) { return a.causal ? max(0, a.Lk - a.Lq + r / a.G + 1) : a.Lk; };
+    const int kb = SPLIT ? (int)blockIdx.y * a.kps : 0;
+    const int ke_all = SPLIT ? min(a.Lk, kb + a.kps) : a.Lk;
+    const int w0 = tile * kRows + 32 * wave;  // the wave's first row
+    // key limits: this lane's row, the wave's smallest and largest, the block's largest
+    const int row = min(w0 + c32, n_rows - 1);
+    const int lim = min(ke_all, limit_of(row));
+    const int lim_lo = min(ke_all, limit_of(min(w0, n_rows - 1)));
+    const int lim_hi = w0 < n_rows ? min(ke_all, limit_of(min(w0 + 31, n_rows - 1))) : 0;
+    const int ke = min(ke_all, limit_of(min(tile * kRows + kRows, n_rows) - 1));
+    const int64_t q_off = ((int64_t)(b * a.Hk * a.G + hk * a.G + row % a.G) * a.Lq + row / a.G) * kDh;
+
+    // q as B fragments: MFMA step kk takes features 16 kk + 8 h .. +8 of the row
+    uint4 qf[QN][8];
+    float c = fabsf(a.scale) * kLog2e;  // the scale's sign goes into q
+    {
+        const float sgn = a.scale < 0.0f ? -1.0f : 1.0f;
+        float qscale = sgn, amax = 0.0f;
+        if constexpr (F16) {
+            for (int kk = 0; kk < 8; kk++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(load_act(a.q, q_off + 16 * kk + 8 * h + e, a.q_dt)));
+            amax = pair32<true>(amax);
+            const int ex = (int)(__float_as_uint(amax) >> 23);
+            const int f = min(max(267 - ex, 1), 253);  // exponent field of 2^(13 - exponent of amax)
+            qscale = sgn * __uint_as_float((uint32_t)f << 23);
+            c *= __uint_as_float((uint32_t)(254 - f) << 23);
+        }
+#pragma unroll
+        for (int kk = 0; kk < 8; kk++) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = load_act(a.q, q_off + 16 * kk + 8 * h + e, a.q_dt) * qscale;
+            uint32_t t[4][QN];
+#pragma unroll
+            for (int p = 0; p < 4; p++) split_pair<F16, QN>(v[2 * p], v[2 * p + 1], t[p]);
+#pragma unroll
+            for (int n = 0; n < QN; n++) qf[n][kk] = make_uint4(t[0][n], t[1][n], t[2][n], t[3][n]);
+        }
+        if (c < 1e-37f) c = 1e-37f;  // a zero scale: equal weights, and masked scores stay -inf
+    }
+
+    floatx16 o[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[t][r] = 0.0f;
+    const float ninf = -__builtin_inff();
+    float m = ninf, l = 0.0f;  // the row's reference maximum (log2 units) and this lane's part of its sum
+
+    const int64_t head = (int64_t)bhk * a.kcap * kDh;
+    const auto rk = make_rsrc(a.k + head, (uint32_t)a.Lk * kDh * 2);  // keys past Lk read 0
+    const auto rv = make_rsrc(a.v + head, (uint32_t)a.Lk * kDh * 2);
+    const int sr = tid >> 4, sc = tid & 15;  // staging: row and 16-byte chunk
+    u32x4_t kr[4], vr[4];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            kr[j] = __builtin_amdgcn_raw_buffer_load_b128(rk, (uint32_t)((k0 + sr + 16 * j) * kDh + 8 * sc) * 2, 0, 0);
+            vr[j] = __builtin_amdgcn_raw_buffer_load_b128(rv, (uint32_t)((k0 + 4 * sr + j) * kDh + 8 * sc) * 2, 0, 0);
+        }
+    };
+    auto stage = [&](uint8_t* buf) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int k = sr + 16 * j;
+            *reinterpret_cast<u32x4_t*>(buf + k * 256 + 16 * (sc ^ (k & 15))) = kr[j];
+        }
+        uint8_t* const vt = buf + kTileBytes;
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            // features 8 sc + 2 d and + 1 of keys 4 sr .. + 3
+            const uint32_t r0 = vr[0][d], r1 = vr[1][d], r2 = vr[2][d], r3 = vr[3][d];
+            const int f = 8 * sc + 2 * d;
+            const int at = 8 * (sr ^ ((f >> 1) & 15));
+            *reinterpret_cast<uint2*>(vt + f * 128 + at) =
+                make_uint2(__builtin_amdgcn_perm(r1, r0, 0x05040100u), __builtin_amdgcn_perm(r3, r2, 0x05040100u));
+            *reinterpret_cast<uint2*>(vt + (f + 1) * 128 + at) =
+                make_uint2(__builtin_amdgcn_perm(r1, r0, 0x07060302u), __builtin_amdgcn_perm(r3, r2, 0x07060302u));
+        }
+    };
+    auto compute = [&](const uint8_t* buf, int k0) {
+        floatx16 s[2];
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[g][r] = 0.0f;
+            const uint8_t* const kt = buf + (32 * g + c32) * 256;
+#pragma unroll
+            for (int kk = 0; kk < 8; kk++) {
+                const uint4 kf = *reinterpret_cast<const uint4*>(kt + 16 * ((2 * kk + h) ^ (c32 & 15)));
+#pragma unroll
+                for (int n = QN - 1; n >= 0; n--) s[g] = mfma<F16>(kf, qf[n][kk], s[g]);
+            }
+        }
+        // register r of s[g] is key k0 + 32 g + 8 (r / 4) + 4 h + r % 4
+        if (k0 + kKeys > lim_lo) {
+#pragma unroll
+            for (int g = 0; g < 2; g++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    if (k0 + 32 * g + 8 * (r >> 2) + 4 * h + (r & 3) >= lim) s[g][r] = ninf;
+        }
+        float mt = ninf;
+#pragma unroll
+        for (int r = 0; r < 16; r++) mt = fmaxf(mt, fmaxf(s[0][r], s[1][r]));
+        mt = pair32<true>(mt) * c;
+        if (__any(mt > m + kLazy)) {
+            const float mn = fmaxf(m, mt);
+            const float f = mn == ninf ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            l *= f;
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) o[t][r] *= f;
+            m = mn;
+        }
+        const float neg = m == ninf ? 0.0f : kPShift - m;
+        float ls = 0.0f;
+#pragma unroll
+        for (int g = 0; g < 2; g++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                s[g][r] = __builtin_amdgcn_exp2f(fmaf(s[g][r], c, neg));
+                ls += s[g][r];
+            }
+        l += ls;
+        const uint8_t* const vt = buf + kTileBytes;
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+            // B: keys 16 kk + 4 h + 0..3, then 16 kk + 8 + 4 h + 0..3
+            const int g = kk >> 1, r0 = 8 * (kk & 1);
+            uint32_t t[4][PN];
+#pragma unroll
+            for (int p = 0; p < 4; p++) split_pair<F16, PN>(s[g][r0 + 2 * p], s[g][r0 + 2 * p + 1], t[p]);
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+                const int f = 32 * d + c32, x = (f >> 1) & 15;
+                const uint2 lo = *reinterpret_cast<const uint2*>(vt + f * 128 + 8 * ((4 * kk + h) ^ x));
+                const uint2 hi = *reinterpret_cast<const uint2*>(vt + f * 128 + 8 * ((4 * kk + 2 + h) ^ x));
+                const uint4 vf = make_uint4(lo.x, lo.y, hi.x, hi.y);
+#pragma unroll
+                for (int n = PN - 1; n >= 0; n--)
+                    o[d] = mfma<F16>(vf, make_uint4(t[0][n], t[1][n], t[2][n], t[3][n]), o[d]);
+            }
+        }
+    };
+
+    if (kb < ke) {
+        load(kb);
+        stage(lds);
+        if (kb + kKeys < ke) load(kb + kKeys);
+        __syncthreads();
+        int slot = 0;
+        for (int k0 = kb; k0 < ke; k0 += kKeys, slot ^= 1) {
+            // LDS slot `slot` holds this tile, the registers the next one
+            if (k0 + kKeys < ke) stage(lds + (slot ^ 1) * 2 * kTileBytes);
+            if (k0 + 2 * kKeys < ke) load(k0 + 2 * kKeys);
+            if (k0 < lim_hi) compute(lds + slot * 2 * kTileBytes, k0);
+            __syncthreads();
+        }
+    }
+
+    l = pair32<false>(l);
+    // lane (h, row) holds features 32 t + 8 (r / 4) + 4 h + r % 4
+    bool bad = !finite(l);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) bad |= !finite(o[t][r]);
+    const uint64_t votes = __ballot(bad && w0 + c32 < n_rows);
+    uint32_t again = (uint32_t)votes | (uint32_t)(votes >> 32);  // rows of the wave to compute again
+    const int64_t grow = (int64_t)bhk * n_rows;
+    if (w0 + c32 < n_rows && !((again >> c32) & 1u)) {
+        if constexpr (SPLIT) {
+            float* const po = a.part_o + ((grow + row) * a.nsplit + blockIdx.y) * kDh;
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    *reinterpret_cast<float4*>(po + 32 * t + 8 * g + 4 * h) =
+                        make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
+            if (h == 0)
+                *reinterpret_cast<float2*>(a.part_ml + ((grow + row) * a.nsplit + blockIdx.y) * 2) = make_float2(m, l);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const int64_t at = q_off + 32 * t + 8 * g + 4 * h;
+                    const float x = o[t][4 * g] / l, y = o[t][4 * g + 1] / l, z = o[t][4 * g + 2] / l,
+                                w = o[t][4 * g + 3] / l;
+                    if (a.out_dt == JH_F32)
+                        *reinterpret_cast<float4*>(static_cast<float*>(a.out) + at) = make_float4(x, y, z, w);
+                    else
+                        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + at) =
+                            make_uint2(pack_bf16x2(x, y), pack_bf16x2(z, w));
+                }
+        }
+    }
+    // rows with a result that is not finite: sdpa_rows_kernel's arithmetic over
+    // the block's keys, one row of the wave at a time
+    while (again) {
+        const int j = __ffs(again) - 1;
+        again &= again - 1;
+        const int r = w0 + j, lj = min(ke_all, limit_of(r));
+        const int64_t at = ((int64_t)(b * a.Hk * a.G + hk * a.G + r % a.G) * a.Lq + r / a.G) * kDh;
+        auto widen = [&](uint16_t v) { return F16 ? f16_to_f32(v) : bf16_to_f32(v); };
+        auto score = [&](int key) {
+            float s = 0.0f;
+            for (int d = 0; d < kDh; d++)
+                s = fmaf(load_act(a.q, at + d, a.q_dt), widen(a.k[head + (int64_t)key * kDh + d]), s);
+            return s * a.scale;
+        };
+        float mx = ninf;
+        for (int key = kb + lane; key < lj; key += 64) mx = fmaxf(mx, score(key));
+        mx = wave_max(mx);
+        float ls = 0.0f, x0 = 0.0f, x1 = 0.0f;
+        for (int k0 = kb; k0 < lj; k0 += 64) {
+            const float e = k0 + lane < lj ? (float)exp((double)(score(k0 + lane) - mx)) : 0.0f;
+            ls += e;
+            for (int jj = 0; jj < min(64, lj - k0); jj++) {
+                const float p = __shfl(e, jj, 64);
+                const uint16_t* const vp = a.v + head + (int64_t)(k0 + jj) * kDh;
+                x0 = fmaf(p, widen(vp[lane]), x0);
+                x1 = fmaf(p, widen(vp[lane + 64]), x1);
+            }
+        }
+        ls = wave_sum(ls);
+        if constexpr (SPLIT) {
+            float* const po = a.part_o + ((grow + r) * a.nsplit + blockIdx.y) * kDh;
+            po[lane] = x0;
+            po[lane + 64] = x1;
+            // (m, l) of the row in the units of the others: no 2^7 on p here
+            if (lane == 0) {
+                a.part_ml[((grow + r) * a.nsplit + blockIdx.y) * 2] = mx * kLog2e + kPShift;
+                a.part_ml[((grow + r) * a.nsplit + blockIdx.y) * 2 + 1] = ls;
+            }
+        } else {
+            store_y(a.out, at + lane, x0 / ls, a.out_dt);
+            store_y(a.out, at + lane + 64, x1 / ls, a.out_dt);
+        }
+    }
+}
+
+// The splits of one row added in split order (one wave per row).
+__global__ __launch_bounds__(256) void sdpa_mfma_merge_kernel(const float* __restrict__ part_o,
+                                                              const float* __restrict__ part_ml, int64_t rows,
+                                                              int n_rows, int G, int Lq, int nsplit,
+                                                              void* __restrict__ out, int out_dt) {
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    const int64_t bhk = row / n_rows;
+    const int r = (int)(row - bhk * n_rows);
+    const float* const ml = part_ml + row * nsplit * 2;
+    float mx = -__builtin_inff();
+    for (int s = 0; s < nsplit; s++) mx = fmaxf(mx, ml[2 * s]);
+    float l = 0.0f, x0 = 0.0f, x1 = 0.0f;
+    for (int s = 0; s < nsplit; s++) {
+        const float m = ml[2 * s];
+        if (m == -__builtin_inff() && ml[2 * s + 1] == 0.0f) continue;  // no keys of the row in this split
+        const float w = m == mx ? 1.0f : __builtin_amdgcn_exp2f(m - mx);
+        const float2 o = *reinterpret_cast<const float2*>(part_o + (row * nsplit + s) * kDh + 2 * lane);
+        l = fmaf(ml[2 * s + 1], w, l);
+        x0 = fmaf(o.x, w, x0);
+        x1 = fmaf(o.y, w, x1);
+    }
+    const int64_t at = ((bhk * G + r % G) * Lq + r / G) * kDh + 2 * lane;
+    store_y(out, at, x0 / l, out_dt);
+    store_y(out, at + 1, x1 / l, out_dt);
+}
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+}  // namespace
+
+// Calls the matrix-core kernel takes; others run sdpa_rows_kernel. Its loads
+// and stores are 16 bytes wide (buffers so aligned) with 32-bit offsets inside
+// a head. fp32 keys and values (no model's caches hold them) stay there.
+bool sdpa_mfma_ok(const void* q, int q_dt, const void* k, const void* v, int kv_dt, const void* out, int64_t B,
+                  int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int64_t Dh) {
+    return Dh == kDh && Lq > 1 && Lk > 0 && (kv_dt == JH_BF16 || kv_dt == JH_F16) &&
+           (q_dt == JH_BF16 || q_dt == JH_F32) && Lk < ((int64_t)1 << 22) && Hq / Hk * Lq < ((int64_t)1 << 30) &&
+           B * Hk * ((Hq / Hk * Lq + kRows - 1) / kRows) < ((int64_t)1 << 30) && aligned16(q) && aligned16(k) &&
+           aligned16(v) && aligned16(out);
+}
+
+// Splits of the keys: one while the row tiles fill the GPU (two blocks per CU);
+// fewer tiles take enough splits to fill it, at least 256 keys each.
+int64_t sdpa_mfma_splits(int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int num_cus) {
+    const int64_t blocks = B * Hk * ((Hq / Hk * Lq + kRows - 1) / kRows);
+    return std::max<int64_t>(1, std::min<int64_t>(2 * (int64_t)num_cus / blocks, Lk / 256));
+}
+
+size_t sdpa_mfma_workspace_bytes(int64_t B, int64_t Hq, int64_t Lq, int64_t nsplit) {
+    return nsplit > 1 ? sizeof(float) * (size_t)(B * Hq * Lq * nsplit) * (kDh + 2) : 0;
+}
+
+Status launch_sdpa_mfma(const void* q, int q_dt, const void* k, const void* v, int kv_dt, void* out, int out_dt,
+                        int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int64_t kcap, float scale,
+                        bool causal, int64_t nsplit, void* workspace, hipStream_t st) {
+    const int64_t G = Hq / Hk, tiles = (G * Lq + kRows - 1) / kRows, rows = B * Hq * Lq;
+    SdpaArgs a{};
+    a.q = q, a.q_dt = q_dt;
+    a.k = static_cast<const uint16_t*>(k), a.v = static_cast<const uint16_t*>(v);
+    a.out = out, a.out_dt = out_dt;
+    a.Hk = (int)Hk, a.G = (int)G, a.Lq = (int)Lq, a.Lk = (int)Lk, a.n_tiles = (int)tiles, a.BHk = (int)(B * Hk);
+    a.kcap = kcap;
+    a.scale = scale;
+    a.causal = causal ? 1 : 0;
+    a.kps = (int)(((Lk + nsplit - 1) / nsplit + kKeys - 1) / kKeys * kKeys);
+    a.nsplit = (int)nsplit;
+    a.part_o = static_cast<float*>(workspace);
+    a.part_ml = a.part_o + (nsplit > 1 ? rows * nsplit * kDh : 0);
+    const dim3 grid((unsigned)(tiles * B * Hk), (unsigned)nsplit);
+    auto go = [&](auto one, auto many) {
+        if (nsplit > 1) hipLaunchKernelGGL(many, grid, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL(one, grid, dim3(256), 0, st, a);
+    };
+    const bool qf = q_dt == JH_F32;
+    if (kv_dt == JH_F16)
+        qf ? go(sdpa_mfma_kernel<true, 2, false>, sdpa_mfma_kernel<true, 2, true>)
+           : go(sdpa_mfma_kernel<true, 1, false>, sdpa_mfma_kernel<true, 1, true>);
+    else
+        qf ? go(sdpa_mfma_kernel<false, 3, false>, sdpa_mfma_kernel<false, 3, true>)
+           : go(sdpa_mfma_kernel<false, 1, false>, sdpa_mfma_kernel<false, 1, true>);
+    if (nsplit > 1)
+        hipLaunchKernelGGL(sdpa_mfma_merge_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, a.part_o,
+                           a.part_ml, rows, (int)(G * Lq), (int)G, (int)Lq, (int)nsplit, out, out_dt);
+    return Status::ok();
+}
+
+}  // namespace jh

@@ -12,8 +12,9 @@
 // SDPA with one query row per head (decode) is split over the key sequence
 // (flash-decoding): block (b*Hk + hk, split) scores its key range for all
 // Hq/Hk query heads of kv head hk with an online softmax and writes (max, sum,
-// weighted values); a second launch merges the splits. Other shapes take a
-// per-query-row kernel with the offset causal mask.
+// weighted values); a second launch merges the splits. Several query rows of
+// head_dim 128 over bf16 or f16 keys run on the matrix cores (attention.hip),
+// other shapes a per-query-row kernel with the offset causal mask.
 #include "jh_common.hpp"
 #include "qmv_tile.hpp"
 

@@ -744,6 +744,20 @@ int jh_sdpa(jh_ctx* c, const void* q, jh_dtype q_dtype, const void* k, const voi
     const bool fast = jh::sdpa_decode_ok(q_dtype, kv_dtype, Hq, Hk, Lq, Dh);
     if (fast && (!aligned16(k) || !aligned16(v)))
         return fail(c, JH_ERR_INVALID, std::string(op) + ": k and v must be 16-byte aligned");
+    if (jh::sdpa_mfma_ok(q, q_dtype, k, v, kv_dtype, out, B, Hq, Hk, Lq, Lk, Dh)) {
+        // a split of the keys needs a workspace; where it cannot grow (a stream
+        // under capture, no memory) the call runs unsplit
+        int64_t nsplit = jh::sdpa_mfma_splits(B, Hq, Hk, Lq, Lk, c->num_cus);
+        if (ensure_workspace(c, jh::sdpa_mfma_workspace_bytes(B, Hq, Lq, nsplit), op) != JH_OK) {
+            c->err.clear();
+            nsplit = 1;
+        }
+        if (int r = finish(c, jh::launch_sdpa_mfma(q, q_dtype, k, v, kv_dtype, out, out_dtype, B, Hq, Hk, Lq, Lk,
+                                                   kv_capacity, scale, causal != 0, nsplit, c->ws, c->stream),
+                           op))
+            return r;
+        return check_values(c, op, out, out_dtype, B * Hq * Lq * Dh);
+    }
     const size_t need = jh::sdpa_workspace_bytes(q_dtype, kv_dtype, B, Hq, Hk, Lq, Lk, Dh, c->num_cus);
     if (need)
         if (int r = ensure_workspace(c, need, op)) return r;

@@ -1,0 +1,123 @@
+"""SDPA with several query rows per head on the matrix cores (attention.hip),
+against the CPU oracle at the sizes where its tiles end.
+
+Bar 1e-5 of max|oracle| for fp32 results: both sides sum a score's 128 products
+in fp32, so a score of |s| <= 8 is off by up to about sqrt(128) * 2^-24 * 8 =
+5e-6 on each side, which is the relative error of that key's weight. bf16
+results add their own rounding, half a unit of an 8-bit significand: 2^-8.
+"""
+import numpy as np
+import pytest
+
+from janis_amd import synth
+from janis_amd.engine import BF16, F16, F32
+from tests.conftest import Graph, rel_ok, step
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+def _put(hip, a, dt):
+    a = np.asarray(a, np.float32)
+    if dt == BF16:
+        return hip.FromBF16Bits(synth.f32_to_bf16_bits(a), *a.shape)
+    if dt == F16:
+        return hip.FromRaw(F16, a.astype(np.float16), *a.shape)
+    return hip.FromFloats(a, *a.shape)
+
+
+def _round(a, dt):
+    if dt == BF16:
+        return synth.bf16_bits_to_f32(synth.f32_to_bf16_bits(a))
+    return a.astype(np.float16).astype(np.float32) if dt == F16 else a
+
+
+def _case(B, Hq, Hk, Lq, Lk, q_dt, kv_dt, spread=1.5):
+    rng = np.random.default_rng(Lq * 1009 + Lk * 7 + Hq)
+    q = _round((spread * rng.standard_normal((B, Hq, Lq, D))).astype(np.float32), q_dt)
+    k = _round((spread * rng.standard_normal((B, Hk, Lk, D))).astype(np.float32), kv_dt)
+    v = _round(rng.standard_normal((B, Hk, Lk, D)).astype(np.float32), kv_dt)
+    return q, k, v
+
+
+def _cache(hip, a, dt, cap):
+    """a's rows at the start of a [B, H, cap, D] buffer whose other rows are NaN."""
+    B, H, L, _ = a.shape
+    full = np.full((B, H, cap, D), np.nan, np.float32)
+    full[:, :, :L] = a
+    return _put(hip, full, dt)
+
+
+# rows of a kv head (Hq / Hk * Lq) and keys around the wave's 32, the block's 128
+# and the key tile's 64; several blocks; calls split over the keys (Lk >= 512
+# with few rows); group sizes that are no power of two; a batch
+@pytest.mark.parametrize("B,Hq,Hk,Lq,Lk,causal", [
+    (1, 2, 2, 2, 2, True), (1, 1, 1, 32, 64, True), (1, 1, 1, 33, 65, True), (1, 4, 1, 32, 63, False),
+    (2, 6, 2, 43, 129, True), (1, 8, 8, 127, 128, True), (1, 5, 1, 26, 191, False), (1, 16, 2, 7, 1025, True),
+    (1, 8, 8, 3, 512, False), (1, 4, 4, 200, 700, True)])
+@pytest.mark.parametrize("q_dt,kv_dt", [(F32, F16), (BF16, F16), (F32, BF16), (BF16, BF16)])
+def test_sdpa_mfma(hip, oracle, B, Hq, Hk, Lq, Lk, causal, q_dt, kv_dt):
+    q, k, v = _case(B, Hq, Hk, Lq, Lk, q_dt, kv_dt)
+    kc, vc = _cache(hip, k, kv_dt, Lk + 5), _cache(hip, v, kv_dt, Lk + 5)
+    step(f"jh_sdpa rows B={B} Hq={Hq} Hk={Hk} Lq={Lq} Lk={Lk} causal={causal} q={q_dt} kv={kv_dt}")
+    want = oracle.sdpa(q, k, v, D ** -0.5, causal)
+    for out_dt, bar in ((F32, 1e-5), (BF16, 2.0 ** -8 + 1e-5)):
+        got = hip.Floats(hip.SDPA(_put(hip, q, q_dt), kc, vc, D ** -0.5, causal, kv_len=Lk, out_dtype=out_dt))
+        ok, dd, sc = rel_ok(got, want, bar)
+        assert ok, (out_dt, dd, sc)
+
+
+@pytest.mark.parametrize("scale,bar", [(0.0, 1e-5), (1e-3, 1e-5), (-0.1, 1.4e-4), (3.0, 7e-4)])
+def test_sdpa_mfma_scales(hip, oracle, scale, bar):
+    """The scale's sign and size, rows of q of very different sizes (a row's own
+    power of two for f16 keys) and scores far apart: scores of up to 100 (scale
+    -0.1) and 500 (scale 3) are off by sqrt(128) * 2^-24 times that, 7e-5 and
+    3.4e-4, on each side."""
+    q, k, v = _case(1, 2, 1, 20, 90, F32, F16)
+    q *= (10.0 ** np.linspace(-6, 1, 20, dtype=np.float32))[None, None, :, None] * (1.0 if scale < 1 else 0.1)
+    step(f"jh_sdpa rows scale={scale}")
+    got = hip.Floats(hip.SDPA(_put(hip, q, F32), _put(hip, k, F16), _put(hip, v, F16), scale, True))
+    ok, dd, sc = rel_ok(got, oracle.sdpa(q, k, v, scale, True), bar)
+    assert ok, (dd, sc)
+
+
+@pytest.mark.parametrize("kv_dt", [F16, BF16])
+@pytest.mark.parametrize("Lk", [100, 600])
+def test_sdpa_mfma_values_not_finite(hip, oracle, Lk, kv_dt):
+    """An infinity or NaN in a key or value row reaches the rows that attend to
+    it and no other, also inside one tile and one split."""
+    Lq = 40
+    q, k, v = _case(1, 4, 2, Lq, Lk, F32, kv_dt)
+    v[0, 0, Lk - 10, 3] = np.inf   # seen by the last 10 queries of kv head 0
+    v[0, 1, Lk - 20, 7] = np.nan   # ... the last 20 of kv head 1
+    k[0, 1, Lk - 5, 9] = np.nan    # ... the last 5: all their features
+    step(f"jh_sdpa rows, values not finite, Lk={Lk}")
+    got = hip.Floats(hip.SDPA(_put(hip, q, F32), _put(hip, k, kv_dt), _put(hip, v, kv_dt), D ** -0.5, True))
+    with np.errstate(all="ignore"):
+        want = oracle.sdpa(q, k, v, D ** -0.5, True)
+    assert np.isposinf(want[0, :2, Lq - 10:, 3]).all() and np.isnan(want[0, 2:, Lq - 20:, 7]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    fine = np.isfinite(want)
+    ok, dd, sc = rel_ok(got[fine], want[fine], 1e-5)
+    assert ok, (dd, sc)
+
+
+def test_sdpa_mfma_captured_without_workspace(oracle):
+    """A call that would split its keys still captures on a context whose
+    workspace was never sized (it runs unsplit), and replays to its result."""
+    from janis_amd.engine import HipBackend
+
+    b = HipBackend(0)
+    q, k, v = _case(1, 4, 2, 9, 1500, F32, F16)
+    Q, K, V = _put(b, q, F32), _put(b, k, F16), _put(b, v, F16)
+    arena = b.make_arena(1 << 20)
+    out = []
+    with b.use_arena(arena):
+        step("jh_sdpa rows captured first")
+        g = Graph(b, lambda: out.append(b.SDPA(Q, K, V, D ** -0.5, True)))
+    want = oracle.sdpa(q, k, v, D ** -0.5, True)
+    for _ in range(3):
+        g.replay()
+        ok, dd, sc = rel_ok(b.Floats(out[-1]), want, 1e-5)
+        assert ok, (dd, sc)
+    b.Close()
