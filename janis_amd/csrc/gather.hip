@@ -371,6 +371,274 @@ __global__ __launch_bounds__(256) void moe_qmv_kernel(MoeArgs a) {
     }
 }
 
+// ---- many pairs per expert: the bucket's pairs on the matrix cores -----------------
+//
+// The dot products above read each weight once per bucket but multiply it once
+// per pair with VALU instructions, which bounds them from a few pairs per expert
+// on. Here a block of 4 waves takes up to 64 pairs of a bucket (the A operand,
+// rows of x in LDS) against 32 rows of each weight stack per wave (the B operand,
+// unpacked in registers) with v_mfma_f32_32x32x16_bf16, in K steps of 256.
+//
+// Nothing is rounded to 16 bits that the dot products do not round. Codes enter
+// as exact bf16: a byte holding a 4-bit code q, read as e4m3, is q * 2^-9 for
+// every q (subnormal and normal alike), so v_cvt_scalef32_pk_bf16_fp8 with scale
+// 512 makes two of them bf16 q, in the order q0 q2 q4 q6 q1 q3 q5 q7 of a word
+// split into even and odd nibbles; x is stored in that order. A 64-wide block's
+// sum of products accumulates in fp32 from 0 and meets its scale in fp32 (held by
+// the lane: a lane's accumulators all belong to one weight row). The biases come
+// as one more product per step, sum(x) of each block times its bias: sum(x),
+// taken in fp32 as x is staged, enters as three bf16 terms (24 bits), bf16 biases
+// as they are, f16 ones as two terms. One MFMA covers k of one block only: lane
+// half h of MFMA j of block g supplies word 8 g + 4 h + j of its weight row.
+//
+// Bound: HBM up to about 64 pairs per expert (each routed expert's weights are
+// read once per 64 pairs). So the weight loads are whole 128-byte lines, a wave's
+// 32 rows of a step per stack as 4 loads into LDS of 8 rows each, and a step's
+// weights move from LDS to registers at once, so that the next step's loads are
+// in flight in the same space during its MFMAs; two blocks per CU. At 500 tokens
+// (31 pairs per expert of 2048 x 768) gate + up took 98 us and down 58 us, the
+// dot products 636 and 426; what holds it there is the issue of VALU (the scaling
+// and unpacking, about 44 instructions per 32 x 32 block of 64 k), LDS reads and
+// MFMAs together at two waves per SIMD, not one of them.
+typedef float moe_f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 moe_bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kMfmaRows = 64;
+
+// The 8 codes of a word as bf16, in the order q0 q2 q4 q6 q1 q3 q5 q7.
+__device__ __forceinline__ moe_bf16x8 code_frag(uint32_t word) {
+    const uint32_t lo = word & 0x0F0F0F0Fu, hi = (word >> 4) & 0x0F0F0F0Fu;
+    auto two = [](uint32_t w, auto sel) {
+        return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 512.0f, decltype(sel)::value));
+    };
+    return __builtin_bit_cast(moe_bf16x8, make_uint4(two(lo, std::false_type{}), two(lo, std::true_type{}),
+                                                     two(hi, std::false_type{}), two(hi, std::true_type{})));
+}
+
+template <int EPI, bool SB_F16, int GSL>
+__global__ __launch_bounds__(256, 2) void moe_mfma_kernel(MoeArgs a, uint32_t K) {
+    constexpr int NSTK = EPI == EPI_SWIGLU ? 2 : 1;
+    typedef uint32_t sb_t __attribute__((ext_vector_type(2)));  // a lane's scales (or biases) of a step
+    __shared__ __attribute__((aligned(16))) uint8_t xs[kMfmaRows * 512];
+    __shared__ __attribute__((aligned(16))) uint8_t ws[4 * NSTK * 4096];
+    // sum(x) of a row's four 64-wide blocks as bf16 terms: high, middle, low, 0
+    __shared__ __attribute__((aligned(16))) uint2 xsum[kMfmaRows][4];
+    __shared__ __attribute__((aligned(16))) int sp[kMfmaRows];  // a tile's pairs,
+    __shared__ int sx[kMfmaRows];                               // their rows of x
+    __shared__ __attribute__((aligned(16))) float ssc[kMfmaRows];  // and scores (EPI_PARTIAL)
+    // (entries past the used experts are in bounds: read together, one round trip)
+    const int U = a.ws[0];
+    const int64_t e = a.ws[1 + blockIdx.y];
+    const int p_begin = a.ws[1 + a.E + blockIdx.y], p_end = a.ws[2 + a.E + blockIdx.y];
+    if ((int)blockIdx.y >= U) return;
+    const int* const pairs = a.ws + 2 + 2 * a.E;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t N = a.N, P = K >> 3, G = K >> GSL;
+    const int nsteps = (int)(K >> 8);
+    const auto rx = make_rsrc(a.x, (uint32_t)(a.n_pairs / (a.a_vectors == 1 ? (int)a.k_slots : 1)) * K * 2);
+    __amdgpu_buffer_rsrc_t rw[NSTK], rs[NSTK], rb[NSTK];
+#pragma unroll
+    for (int t = 0; t < NSTK; t++) {
+        rw[t] = make_rsrc(a.w[t] + e * (int64_t)N * P, N * P * 4);
+        rs[t] = make_rsrc(a.s[t] + e * (int64_t)N * G, N * G * 2);
+        rb[t] = make_rsrc(a.b[t] + e * (int64_t)N * G, N * G * 2);
+    }
+    // One tile of up to 32 * MT pairs of the bucket from m0.
+    auto tile = [&](int m0, auto mt) {
+        constexpr int MT = decltype(mt)::value;
+        constexpr int NXC = 4 * MT;  // 16-byte chunks of x per thread and step
+        const int live = min(32 * MT, p_end - m0);
+        // opaque per tile: or the addresses of every tile's stores are computed
+        // ahead of the loop over tiles, and spilled
+        int lane_t = lane;
+        asm volatile("" : "+v"(lane_t));
+        const int h = lane_t >> 5, c32 = lane_t & 31;
+        const uint32_t n0 = blockIdx.x * 128 + wave * 32, n = n0 + c32;  // this lane's weight row of each stack
+        // Steps past the last repeat its loads, so that the loop has no branch (the
+        // compiler would sink the accumulators' updates past it and spill).
+        auto step_k0 = [&](int step) { return (uint32_t)min(step, nsteps - 1) * 256; };
+        auto load_w = [&](int step) {
+            const uint32_t k0 = step_k0(step);
+#pragma unroll
+            for (int t = 0; t < NSTK; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int r = 8 * i + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+                    lds_load16(rw[t], ((n0 + r) * P + 4 * c) * 4, (k0 >> 3) * 4,
+                               lds_addr(ws + (wave * NSTK + t) * 4096 + 1024 * i));
+                }
+        };
+        load_w(0);
+        __syncthreads();  // the last tile's readers of sp and x are done
+        if (tid < 32 * MT) {
+            const int pair = pairs[m0 + min(tid, live - 1)];  // past the last: a repeat
+            sp[tid] = pair;
+            sx[tid] = a.a_vectors == 1 ? pair / (int)a.k_slots : pair;
+            if constexpr (EPI == EPI_PARTIAL) ssc[tid] = a.scores[pair];
+        }
+        __syncthreads();
+        uint32_t xoff[NXC];  // this thread's chunk of x in row tid / 32 + 8 j
+#pragma unroll
+        for (int j = 0; j < NXC; j++) xoff[j] = ((uint32_t)sx[(tid >> 5) + 8 * j] * K + 8 * (tid & 31)) * 2;
+        uint4 xr[NXC];
+        sb_t sr[NSTK], br[NSTK];
+        auto load_x = [&](int step) {
+            const uint32_t k0 = step_k0(step);
+#pragma unroll
+            for (int j = 0; j < NXC; j++) {
+                const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff[j] + 2 * k0, 0, 0);
+                xr[j] = make_uint4(v.x, v.y, v.z, v.w);
+            }
+#pragma unroll
+            for (int t = 0; t < NSTK; t++) {
+                const uint32_t off = (n * G + (k0 >> GSL)) * 2;
+                if constexpr (GSL == 6) {
+                    sr[t] = __builtin_amdgcn_raw_buffer_load_b64(rs[t], off, 0, 0);
+                    br[t] = __builtin_amdgcn_raw_buffer_load_b64(rb[t], off, 0, 0);
+                } else {
+                    sr[t].x = __builtin_amdgcn_raw_buffer_load_b32(rs[t], off, 0, 0);
+                    br[t].x = __builtin_amdgcn_raw_buffer_load_b32(rb[t], off, 0, 0);
+                }
+            }
+        };
+        auto stage = [&]() {
+#pragma unroll
+            for (int j = 0; j < NXC; j++) {
+                const int row = (tid >> 5) + 8 * j, c = tid & 31;
+                const uint4 v = xr[j];
+                float sum = dot2_bf16(v.y, kBf16Ones, dot2_bf16(v.x, kBf16Ones, 0.0f)) +
+                            dot2_bf16(v.w, kBf16Ones, dot2_bf16(v.z, kBf16Ones, 0.0f));
+                // over the 8 lanes of the 64-wide block
+                auto dpp = [](float f, auto ctrl) {
+                    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, f),
+                                                                                 decltype(ctrl)::value, 0xF, 0xF, false));
+                };
+                sum += dpp(sum, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+                sum += dpp(sum, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+                sum += dpp(sum, std::integral_constant<int, 0x141>{});  // row_half_mirror
+                *reinterpret_cast<uint4*>(xs + row * 512 + 16 * (c ^ (row & 15))) =
+                    make_uint4(__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u),
+                               __builtin_amdgcn_perm(v.y, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.z, 0x07060302u));
+                const uint16_t hi = f32_to_bf16_hw(sum);
+                const float r1 = sum - bf16_to_f32(hi);
+                const uint16_t mid = f32_to_bf16_hw(r1);
+                const uint16_t lo = f32_to_bf16_hw(r1 - bf16_to_f32(mid));
+                xsum[row][c >> 3] = make_uint2(hi | ((uint32_t)mid << 16), lo);  // the 8 lanes alike: no branch
+            }
+        };
+        moe_f32x16 acc[NSTK][MT];
+#pragma unroll
+        for (int t = 0; t < NSTK; t++)
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[t][i][r] = 0.0f;
+        // 16 bits of scale or bias block el
+        auto sb_bits = [](const sb_t& v, int el) { return (uint16_t)(v[el >> 1] >> (16 * (el & 1))); };
+        auto widen = [](uint16_t v) { return SB_F16 ? f16_to_f32(v) : bf16_to_f32(v); };
+
+        load_x(0);
+        for (int s = 0; s < nsteps; s++) {
+            __syncthreads();  // every wave is done with the last step's x
+            stage();
+            sb_t sc2[NSTK], bi2[NSTK];
+            uint4 w[NSTK][4];
+            wait_vmem<0>();  // this step's weights (issued before its x)
+#pragma unroll
+            for (int t = 0; t < NSTK; t++) {
+                sc2[t] = sr[t], bi2[t] = br[t];
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    w[t][g] = *reinterpret_cast<const uint4*>(ws + (wave * NSTK + t) * 4096 + 128 * c32 +
+                                                              16 * ((2 * g + h) ^ ((c32 >> 1) & 7)));
+            }
+            __syncthreads();  // x is staged; this wave's weights are in registers
+            load_w(s + 1);
+            load_x(s + 1);
+            // the biases: slots 4 g .. + 3 of the lane half that holds block g
+#pragma unroll
+            for (int t = 0; t < NSTK; t++) {
+                const uint16_t b0 = h ? sb_bits(bi2[t], 128 >> GSL) : sb_bits(bi2[t], 0);
+                const uint16_t b1 = h ? sb_bits(bi2[t], 192 >> GSL) : sb_bits(bi2[t], 64 >> GSL);
+                float f0 = widen(b0), f1 = widen(b1);
+#pragma unroll
+                for (int n2 = 0; n2 < (SB_F16 ? 2 : 1); n2++) {
+                    const uint32_t t0 = f32_to_bf16_hw(f0), t1 = f32_to_bf16_hw(f1);
+                    f0 -= bf16_to_f32((uint16_t)t0), f1 -= bf16_to_f32((uint16_t)t1);
+                    const moe_bf16x8 bb = __builtin_bit_cast(
+                        moe_bf16x8, make_uint4(t0 * 0x10001u, t0 * 0x10001u, t1 * 0x10001u, t1 * 0x10001u));
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+                        acc[t][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            *reinterpret_cast<const moe_bf16x8*>(&xsum[32 * i + c32][2 * h]), bb, acc[t][i], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int i = 0; i < MT; i++) {
+                    const int row = 32 * i + c32;
+                    moe_f32x16 d[NSTK];
+#pragma unroll
+                    for (int t = 0; t < NSTK; t++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++) d[t][r] = 0.0f;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const moe_bf16x8 av = *reinterpret_cast<const moe_bf16x8*>(
+                            xs + row * 512 + 16 * ((8 * g + 4 * h + j) ^ (row & 15)));
+#pragma unroll
+                        for (int t = 0; t < NSTK; t++) {
+                            const uint32_t word = j == 0 ? w[t][g].x : j == 1 ? w[t][g].y : j == 2 ? w[t][g].z : w[t][g].w;
+                            d[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, code_frag(word), d[t], 0, 0, 0);
+                        }
+                    }
+#pragma unroll
+                    for (int t = 0; t < NSTK; t++) {
+                        const float sc = widen(sb_bits(sc2[t], (64 * g) >> GSL));
+#pragma unroll
+                        for (int r = 0; r < 16; r++) acc[t][i][r] = fmaf(sc, d[t][r], acc[t][i][r]);
+                    }
+                }
+        }
+        wait_vmem<0>();  // no load may still target LDS when the tile ends
+        if (n < N) {
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int r0 = 32 * i + 8 * q + 4 * h;
+                    const int4 p4 = *reinterpret_cast<const int4*>(&sp[r0]);
+                    const int pr[4] = {p4.x, p4.y, p4.z, p4.w};
+                    float4 s4 = make_float4(0, 0, 0, 0);
+                    if constexpr (EPI == EPI_PARTIAL) s4 = *reinterpret_cast<const float4*>(&ssc[r0]);
+                    const float sv[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        if (r0 + r >= live) continue;
+                        const int64_t at = (int64_t)pr[r] * N + n;
+                        const float v0 = acc[0][i][4 * q + r];
+                        if constexpr (EPI == EPI_PARTIAL) {
+                            static_cast<float*>(a.y)[at] = sv[r] * v0;
+                        } else {
+                            const float v = EPI == EPI_SWIGLU ? silu(v0) * acc[NSTK - 1][i][4 * q + r] : v0;
+                            if (a.y_dt == JH_BF16)
+                                static_cast<uint16_t*>(a.y)[at] = f32_to_bf16_hw(v);
+                            else
+                                static_cast<float*>(a.y)[at] = v;
+                        }
+                    }
+                }
+        }
+    };
+    for (int m0 = p_begin; m0 < p_end; m0 += kMfmaRows) {
+        if (p_end - m0 > 32) tile(m0, std::integral_constant<int, 2>{});
+        else tile(m0, std::integral_constant<int, 1>{});
+    }
+}
+
 __device__ __forceinline__ void store_out(void* y, int dt, int64_t i, float v) {
     if (dt == JH_BF16)
         static_cast<uint16_t*>(y)[i] = f32_to_bf16_hw(v);
@@ -570,8 +838,33 @@ void run_tile(const MoeArgs& a, bool sb_f16, int mode, int64_t max_u, hipStream_
 
 // Tile per row length P (32-bit words). SWIGLU holds two stacks' rows, so it
 // takes half the rows per wave of the single-stack epilogues.
+// Calls that run the bucket's pairs on the matrix cores: workspace buckets with
+// kMfmaPairsPerExpert pairs per expert of the stack, groups of 64 or 128, every K
+// of the tiles (a multiple of 256), x within a buffer resource's 2 GiB. Measured
+// on MI355X, jh_moe_route + jh_moe_swiglu of 128 experts (2048 x 768, top 8), dot
+// products against matrix cores: 16 tokens 88 / 105 us, 24 109 / 114, 32 126 /
+// 119, 48 159 / 128, 500 1004 / 187, 2000 3831 / 465. The line is at 32 tokens,
+// 2 pairs per expert.
+constexpr int64_t kMfmaPairsPerExpert = 2;
+bool moe_mfma_ok(const MoeArgs& a, int64_t P, int mode) {
+    return mode == MODE_WS && (a.gs_log2 == 6 || a.gs_log2 == 7) && P % 32 == 0 &&
+           a.n_pairs >= kMfmaPairsPerExpert * a.E && (int64_t)a.n_pairs * P * 16 < ((int64_t)1 << 31);
+}
+
+template <int EPI>
+void run_mfma(const MoeArgs& a, int64_t P, bool sb_f16, int64_t max_u, hipStream_t st) {
+    const dim3 grid((unsigned)((a.N + 127) / 128), (unsigned)max_u);
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, a, (uint32_t)(8 * P)); };
+    if (a.gs_log2 == 6) sb_f16 ? go(moe_mfma_kernel<EPI, true, 6>) : go(moe_mfma_kernel<EPI, false, 6>);
+    else sb_f16 ? go(moe_mfma_kernel<EPI, true, 7>) : go(moe_mfma_kernel<EPI, false, 7>);
+}
+
 template <int EPI>
 bool run_fast(const MoeArgs& a, int64_t P, bool sb_f16, int mode, int64_t max_u, hipStream_t st) {
+    if (moe_mfma_ok(a, P, mode)) {
+        run_mfma<EPI>(a, P, sb_f16, max_u, st);
+        return true;
+    }
     constexpr int R4 = EPI == EPI_SWIGLU ? 2 : 4;
     constexpr int R2 = EPI == EPI_SWIGLU ? 1 : 2;
     switch (P) {

@@ -191,6 +191,33 @@ __device__ __forceinline__ float pair_up(uint4 v, uint32_t* xp) {
     return ab + cd;
 }
 
+// ---- loads into LDS -------------------------------------------------------------
+// Issued from inline asm, with explicit waits (wait_vmem): the compiler tracks
+// loads into LDS it issued itself and makes each LDS read wait for all of them.
+// LDS byte offset of a __shared__ address (the value M0 takes for a load into LDS).
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) const void*)p);
+}
+// 16 bytes per lane into LDS at m0 + 16 * lane (the s_nop covers the M0 write).
+__device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t m0) {
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(m0) : "memory");
+}
+// The same with a wave-uniform part of the offset in soff; the range check
+// applies to voff, which carries the row, so rows past the buffer still read 0.
+__device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t m0) {
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r),
+                 "s"(__builtin_amdgcn_readfirstlane(soff)), "{m0}"(m0)
+                 : "memory");
+}
+// 4 bytes per lane into LDS at m0 + 4 * lane.
+__device__ __forceinline__ void lds_load4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t m0) {
+    asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(m0) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_vmem() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 // Load element i of a scale/bias array of the given dtype as fp32 (exact).
 __device__ __forceinline__ float load_sb(const void* p, int64_t i, int dt) {
     if (dt == JH_BF16) return bf16_to_f32(static_cast<const uint16_t*>(p)[i]);

@@ -613,30 +613,6 @@ __global__ __launch_bounds__(64 * NW, 2) void qmm_wreg_kernel(
 // after step t's own leaves exactly those in flight; any load the compiler adds
 // in between only makes the wait longer, never shorter.
 
-// LDS byte offset of a __shared__ address (the value M0 takes for a load into LDS).
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-    return __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) const void*)p);
-}
-// 16 bytes per lane into LDS at m0 + 16 * lane (the s_nop covers the M0 write).
-__device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t m0) {
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(m0) : "memory");
-}
-// The same with a wave-uniform part of the offset in soff; the range check
-// applies to voff, which carries the row, so rows past the buffer still read 0.
-__device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t m0) {
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r),
-                 "s"(__builtin_amdgcn_readfirstlane(soff)), "{m0}"(m0)
-                 : "memory");
-}
-// 4 bytes per lane into LDS at m0 + 4 * lane.
-__device__ __forceinline__ void lds_load4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t m0) {
-    asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(m0) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vmem() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // Dwords of scales (and of biases) per lane per super-step: SUP/2 elements of
 // the lane's K half are NG groups; 0 when they do not fill whole dwords.
 template <int SBT, int GSL>

@@ -1,0 +1,97 @@
+"""Expert products of buckets with many pairs on the matrix cores (gather.hip's
+moe_mfma_kernel) against the CPU oracle, at the sizes where its tiles end.
+
+Bar 1e-5 of max|oracle| for fp32 results of one product: the products of codes
+and bf16 x are exact in fp32 on both sides, 64 .. 2048 of them are summed in
+fp32 in another order: sqrt(2048) * 2^-24 = 2.7e-6 of the sum of magnitudes,
+which is up to four times the largest result here. Through the SwiGLU block h is
+bf16 on the device, so that one takes the parity bar of bf16 results, 1e-2.
+"""
+import numpy as np
+import pytest
+
+from janis_amd import synth
+from janis_amd.engine import BF16, F16, F32
+from tests.conftest import rel_ok, step, upload_quant
+
+pytestmark = pytest.mark.gpu
+
+
+def _upload(hip, q, sb):
+    if sb == BF16:
+        return upload_quant(hip, q), q.s, q.b
+    s, b = q.s.astype(np.float16), q.b.astype(np.float16)
+    w = upload_quant(hip, q)[0]
+    return (w, hip.FromRaw(F16, s, *s.shape), hip.FromRaw(F16, b, *b.shape)), s.astype(np.float32), b.astype(np.float32)
+
+
+def _buckets(sizes, k_slots, seed):
+    """Expert indices [tokens, k_slots] with sizes[e] pairs of expert e, shuffled."""
+    idx = np.concatenate([np.full(n, e, np.int32) for e, n in enumerate(sizes)])
+    np.random.default_rng(seed).shuffle(idx)
+    return idx.reshape(-1, k_slots)
+
+
+# buckets around the tile's 32 and 64 pairs, an unused expert, several tiles of
+# one bucket; rows that are no multiple of a wave's 32 or a block's 128; the
+# shortest K and one that is not a power of two; both groups, both scale types
+@pytest.mark.parametrize("sizes,slots,n,k,gs,sb", [
+    ((1, 31, 32, 0), 4, 128, 256, 64, BF16), ((33, 63, 64, 4), 4, 33, 768, 64, F16),
+    ((65, 0, 130, 1, 4), 8, 100, 512, 128, BF16), ((2, 2, 2, 2, 128), 8, 257, 2048, 64, BF16),
+    ((40, 40), 1, 160, 1536, 128, F16)])
+def test_gather_mfma(hip, oracle, sizes, slots, n, k, gs, sb):
+    E, idx = len(sizes), _buckets(sizes, slots, n + k)
+    q = synth.quant_linear(810 + n, n, k, gs, lead=(E,))
+    (w, s, b), sf, bf = _upload(hip, q, sb)
+    for A in {1, slots}:
+        xb, x = synth.activations(820 + A, (idx.shape[0], A, 1, k))
+        step(f"jh_gather_quant_matmul buckets={sizes} A={A} n={n} k={k} gs={gs} sb={sb}")
+        want = oracle.gather_quant_matmul(x, q.w, sf, bf, idx, gs)
+        X, it = hip.FromBF16Bits(xb, idx.shape[0], A, 1, k), hip.FromInt32(idx)
+        for out_dt, bar in ((F32, 1e-5), (BF16, 2.0 ** -8 + 1e-5)):
+            y = hip.Floats(hip.GatherQuantMatmul(X, w, s, b, it, True, gs, 4, out_dtype=out_dt))
+            ok, d, sc = rel_ok(y, want, bar)
+            assert ok, (A, out_dt, d, sc)
+
+
+@pytest.mark.parametrize("sizes,H,I,gs,out_dtype", [((1, 31, 0, 64), 256, 512, 64, F32),
+                                                    ((65, 7, 96), 1024, 768, 128, BF16)])
+def test_moe_swiglu_mfma(hip, oracle, sizes, H, I, gs, out_dtype):
+    E, slots = len(sizes), 4
+    idx = _buckets(sizes, slots, H)
+    qs = [synth.quant_linear(830 + i + H, *(I, H) if i < 2 else (H, I), gs, lead=(E,)) for i in range(3)]
+    sc = np.random.default_rng(I).random(idx.shape).astype(np.float32)
+    xb, x = synth.activations(831, (idx.shape[0], H))
+    st = [upload_quant(hip, q) for q in qs]
+    args = (hip.FromBF16Bits(xb, *x.shape), *st, hip.FromInt32(idx), hip.FromFloats(sc), gs, 4)
+    step(f"jh_moe_swiglu buckets={sizes} H={H} I={I} gs={gs}")
+    first = hip.Floats(hip.MoeSwiGLU(*args, out_dtype=out_dtype))
+    ok, d, s = rel_ok(first, oracle.moe_apply(x, *[(q.w, q.s, q.b) for q in qs], idx, sc, gs), 1e-2)
+    assert ok, (d, s)
+    again = hip.Floats(hip.MoeSwiGLU(*args, out_dtype=out_dtype))
+    assert np.array_equal(first.view(np.uint32), again.view(np.uint32))
+
+
+def test_gather_mfma_rows_apart(hip, oracle):
+    """A pair whose x holds a NaN or an infinity, and one with an index outside
+    the stack, leave the other pairs of their bucket and tile alone."""
+    E, n, k = 2, 64, 512
+    idx = _buckets((40, 24), 4, 3)
+    q = synth.quant_linear(840, n, k, lead=(E,))
+    w, s, b = upload_quant(hip, q)
+    xb, x = synth.activations(841, (16, 4, 1, k))
+    xb, x = xb.copy(), x.copy()
+    for at, bits in (((3, 1, 0, 5), 0x7FC0), ((9, 2, 0, 300), 0x7F80)):
+        xb[at] = bits
+        x[at] = synth.bf16_bits_to_f32(np.uint16(bits))
+    want = oracle.gather_quant_matmul(x, q.w, q.s, q.b, idx, 64)
+    idx = idx.copy()
+    idx[12, 0] = E
+    step("jh_gather_quant_matmul, rows that are not finite")
+    y = hip.Floats(hip.GatherQuantMatmul(hip.FromBF16Bits(xb, 16, 4, 1, k), w, s, b, hip.FromInt32(idx), True, 64, 4,
+                                         out_dtype=F32))
+    odd = np.zeros((16, 4), bool)
+    odd[3, 1] = odd[9, 2] = odd[12, 0] = True
+    assert not np.isfinite(y[3, 1]).any() and not np.isfinite(y[9, 2]).any() and np.isnan(y[12, 0]).all()
+    ok, d, sc = rel_ok(y[~odd], want[~odd], 1e-5)
+    assert ok, (d, sc)
