@@ -794,21 +794,41 @@ __global__ __launch_bounds__(256) void moe_down_combine_kernel(MoeArgs a, void* 
 
 // out[t, :] = the sum over slots k = 0.. of part[t * K + k, :] in slot order,
 // NaN for a token with an expert index outside [0, E) (its partial rows were
-// never written).
-__global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ part, const int32_t* __restrict__ idx,
+// never written: read, but not added). Four features per thread, eight slots'
+// indices and rows requested together: one memory round trip for top 8 (500 tokens
+// of 2048 on MI355X: 7.5 us against 13.8 with one feature per thread and one slot
+// at a time).
+__global__ __launch_bounds__(128) void moe_combine_kernel(const float* __restrict__ part, const int32_t* __restrict__ idx,
                                                           int64_t n_tok, int64_t K, int64_t E, int64_t H,
                                                           void* __restrict__ out, int out_dt) {
-    const int64_t n = n_tok * H;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t t = i / H, h = i - t * H;
-        float v = 0.0f;
+    const int64_t n4 = n_tok * H / 4;  // H is a multiple of 256
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t t = 4 * i / H, h = 4 * i - t * H;
+        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         bool bad = false;
-        for (int64_t k = 0; k < K; k++) {
-            const int32_t e = idx[t * K + k];
-            if (e < 0 || e >= E) bad = true;
-            else v += part[(t * K + k) * H + h];
+        for (int64_t k0 = 0; k0 < K; k0 += 8) {
+            int32_t e[8];
+            float4 r[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int64_t pair = t * K + min(k0 + j, K - 1);
+                e[j] = idx[pair];
+                r[j] = *reinterpret_cast<const float4*>(part + pair * H + h);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                if (k0 + j >= K) break;
+                if (e[j] < 0 || e[j] >= E) bad = true;
+                else v[0] += r[j].x, v[1] += r[j].y, v[2] += r[j].z, v[3] += r[j].w;
+            }
         }
-        store_out(out, out_dt, i, bad ? __uint_as_float(0x7fc00000u) : v);
+        if (bad) v[0] = v[1] = v[2] = v[3] = __uint_as_float(0x7fc00000u);
+        if (out_dt == JH_BF16)
+            *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + 4 * i) =
+                make_uint2(f32_to_bf16_hw(v[0]) | ((uint32_t)f32_to_bf16_hw(v[1]) << 16),
+                           f32_to_bf16_hw(v[2]) | ((uint32_t)f32_to_bf16_hw(v[3]) << 16));
+        else
+            *reinterpret_cast<float4*>(static_cast<float*>(out) + 4 * i) = make_float4(v[0], v[1], v[2], v[3]);
     }
 }
 
@@ -1036,13 +1056,93 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const void* __restrict__ 
     }
 }
 
+// The same for up to 64 * PER experts, each lane holding experts lane, lane + 64,
+// ... in registers (their probability and their position in the order array), so
+// that a pass of the selection is two wave-wide reductions with no LDS access and
+// no barrier: the largest probability among positions >= i, then the smallest
+// position that holds it. The in-order sum of the exponentials is read from LDS
+// 64 values at a time, the reads of a chunk together. Bound: the latency of that
+// chain. 128 experts, top 8, on MI355X: 4.3 us a launch for one token and 5.6 for
+// 500, where the kernel above (more than 512 experts) takes 9.8 and 10.8.
+template <int PER>
+__global__ __launch_bounds__(64) void moe_route_wave_kernel(const void* __restrict__ logits, int l_dt, int E, int k,
+                                                            int norm, int32_t* __restrict__ idx_out,
+                                                            float* __restrict__ score_out) {
+    __shared__ __attribute__((aligned(16))) float es[64 * PER];
+    const int lane = threadIdx.x;
+    const int64_t t = blockIdx.x;
+    const float ninf = -__builtin_inff();
+    float p[PER];
+    int pos[PER];
+    float mx = ninf;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int i = lane + 64 * j;
+        const int64_t at = t * E + min(i, E - 1);
+        p[j] = l_dt == JH_BF16 ? bf16_to_f32(static_cast<const uint16_t*>(logits)[at])
+                               : static_cast<const float*>(logits)[at];
+        pos[j] = i;
+        if (i < E) mx = fmaxf(mx, p[j]);
+    }
+    mx = wave_max(mx);
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const float e = (float)exp((double)(p[j] - mx));
+        p[j] = lane + 64 * j < E ? e : 0.0f;  // past the last: + 0 leaves the sum as it is
+        es[lane + 64 * j] = p[j];
+    }
+    __syncthreads();
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        float4 v[16];
+#pragma unroll
+        for (int q = 0; q < 16; q++) v[q] = *reinterpret_cast<const float4*>(&es[64 * j + 4 * q]);
+#pragma unroll
+        for (int q = 0; q < 16; q++) sum = (((sum + v[q].x) + v[q].y) + v[q].z) + v[q].w;
+    }
+#pragma unroll
+    for (int j = 0; j < PER; j++) p[j] = lane + 64 * j < E ? p[j] / sum : __builtin_nanf("");  // never the largest
+    float ks = 0.0f;
+    for (int it = 0; it < k; it++) {
+        float bv = ninf;
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+            if (pos[j] >= it) bv = fmaxf(bv, p[j]);
+        bv = wave_max(bv);
+        float bp = ninf;  // minus the position
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+            if (pos[j] >= it && p[j] == bv) bp = fmaxf(bp, -(float)pos[j]);
+        const int bj = bv == ninf ? it : (int)-wave_max(bp);  // nothing to choose (all NaN): the order stays
+        ks += bv == ninf ? __builtin_nanf("") : bv;
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            if (pos[j] == bj) pos[j] = it;
+            else if (pos[j] == it) pos[j] = bj;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < PER; j++)
+        if (pos[j] < k) {
+            idx_out[t * k + pos[j]] = lane + 64 * j;
+            score_out[t * k + pos[j]] = norm && ks > 0.0f ? p[j] / ks : p[j];
+        }
+}
+
 Status launch_moe_route(const void* logits, int l_dt, int64_t n_tok, int E, int k, bool norm, int32_t* idx,
                         float* scores, hipStream_t st) {
     if (n_tok == 0 || k == 0) return Status::ok();
     if (E > kMaxRouteExperts) return Status::fail(JH_ERR_UNSUPPORTED, "moe_route: more than 4096 experts");
     if (n_tok > 0x7fffffff) return Status::fail(JH_ERR_UNSUPPORTED, "moe_route: too many tokens");
-    hipLaunchKernelGGL(moe_route_kernel, dim3((unsigned)n_tok), dim3(64), 0, st, logits, l_dt, E, k, norm ? 1 : 0,
-                       idx, scores);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)n_tok), dim3(64), 0, st, logits, l_dt, E, k, norm ? 1 : 0, idx, scores);
+    };
+    if (E <= 64) go(moe_route_wave_kernel<1>);
+    else if (E <= 128) go(moe_route_wave_kernel<2>);
+    else if (E <= 256) go(moe_route_wave_kernel<4>);
+    else if (E <= 512) go(moe_route_wave_kernel<8>);
+    else go(moe_route_kernel);
     return Status::ok();
 }
 
@@ -1123,9 +1223,9 @@ Status launch_moe_mlp(const MoeMlpArgs& a, void* workspace, hipStream_t st) {
         buckets = reinterpret_cast<int*>(wsp);
     }
     const int64_t n_out = a.n_tok * H;
-    const unsigned out_blocks = (unsigned)std::min<int64_t>((n_out + 255) / 256, 4096);
+    const unsigned out_blocks = (unsigned)std::min<int64_t>((n_out / 4 + 127) / 128, 8192);
     if (n_pairs == 0) {  // every token's sum is empty
-        hipLaunchKernelGGL(moe_combine_kernel, dim3(out_blocks), dim3(256), 0, st, static_cast<const float*>(nullptr),
+        hipLaunchKernelGGL(moe_combine_kernel, dim3(out_blocks), dim3(128), 0, st, static_cast<const float*>(nullptr),
                            a.idx, a.n_tok, (int64_t)0, a.n_experts, H, a.out, a.out_dtype);
         return Status::ok();
     }
@@ -1171,7 +1271,7 @@ Status launch_moe_mlp(const MoeMlpArgs& a, void* workspace, hipStream_t st) {
     d.y_dt = JH_F32;
     if (!run_fast<EPI_PARTIAL>(d, Pd, f16, MODE_WS, max_u, st))
         return Status::fail(JH_ERR_UNSUPPORTED, "moe_swiglu: no tile for the down shape");
-    hipLaunchKernelGGL(moe_combine_kernel, dim3(out_blocks), dim3(256), 0, st, static_cast<const float*>(part),
+    hipLaunchKernelGGL(moe_combine_kernel, dim3(out_blocks), dim3(128), 0, st, static_cast<const float*>(part),
                        a.idx, a.n_tok, a.k_slots, a.n_experts, H, a.out, a.out_dtype);
     return Status::ok();
 }

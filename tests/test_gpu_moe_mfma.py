@@ -95,3 +95,30 @@ def test_gather_mfma_rows_apart(hip, oracle):
     assert not np.isfinite(y[3, 1]).any() and not np.isfinite(y[9, 2]).any() and np.isnan(y[12, 0]).all()
     ok, d, sc = rel_ok(y[~odd], want[~odd], 1e-5)
     assert ok, (d, sc)
+
+
+# the register router at the ends of its sizes (64 * 1, 2, 4, 8 experts, and the
+# first size past them), ties and rows that are not finite included
+@pytest.mark.parametrize("E,k", [(1, 1), (63, 63), (64, 8), (65, 8), (128, 8), (129, 3), (256, 16), (257, 8), (512, 8),
+                                 (513, 8)])
+def test_moe_route_sizes(hip, oracle, E, k):
+    """Bit for bit the CPU path's indices and scores."""
+    rng = np.random.default_rng(E)
+    logits = np.concatenate([rng.standard_normal((3, E)), rng.integers(0, 3, (3, E)), rng.standard_normal((2, E))])
+    logits = logits.astype(np.float32)
+    logits[6, E // 2] = np.nan
+    logits[7, E // 3] = np.inf
+    step(f"jh_moe_route E={E} k={k}")
+    it, st = hip.MoeRoute(hip.FromFloats(logits), k, True)
+    got_i, got_s = hip.Ints(it), hip.Floats(st)
+    for t in range(6):
+        p = oracle.softmax_row(logits[t])
+        i, v = oracle.topk(p, k)
+        total = np.float32(0)
+        for x in v:
+            total = np.float32(total + x)
+        assert np.array_equal(got_i[t], i), t
+        assert np.array_equal(got_s[t].view(np.uint32), (v / total).astype(np.float32).view(np.uint32)), t
+    # a NaN or an infinity makes every probability NaN: nothing is larger than
+    # the first, so the order stays
+    assert np.array_equal(got_i[6:], np.tile(np.arange(k, dtype=np.int32), (2, 1))) and np.isnan(got_s[6:]).all()
