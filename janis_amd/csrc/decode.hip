@@ -93,19 +93,45 @@ __device__ float block_sum256(float v, float* red) {
 }
 
 // ---- RMSNorm -------------------------------------------------------------------
-// A row's elements are loaded into registers in one burst (no load waits on an
-// earlier one), squared and summed, then scaled from the registers: x is read
-// once. Rows of up to 1024 take one wave each (per-head norms), longer rows one
-// block of 256 threads.
+// A row's elements and the weights are requested in one burst, as 32-bit words with
+// no branch on their types (no load waits on an earlier one, nor the weights on the
+// reduction), squared and summed, then scaled from the registers: x is read once.
+// Rows of up to 1024 take one wave each (per-head norms), longer rows one block of
+// 256 threads. One fp32 row of 4096 takes 5.1 us on MI355X, 9.2 with the weights
+// loaded after the sum.
 template <int PER>  // elements per lane (wave kernel) or per thread (block kernel)
-__device__ __forceinline__ void load_row(const void* x, int x_dt, int64_t base, int64_t d, int t, int stride,
-                                         float* v) {
+struct NormRow {
+    uint32_t xw[PER], ww[PER];
+    float v[PER];
+    __device__ __forceinline__ void load(const void* x, int x_dt, int64_t base, const void* w, int w_dt, int64_t d,
+                                         int t, int stride) {
 #pragma unroll
-    for (int e = 0; e < PER; e++) {
-        const int64_t i = t + (int64_t)e * stride;
-        v[e] = i < d ? ld_act(x, base + i, x_dt) : 0.0f;
+        for (int e = 0; e < PER; e++) {
+            const int64_t i = min(t + (int64_t)e * stride, d - 1);
+            xw[e] = ld_word(x, base + i, x_dt);
+            ww[e] = ld_word(w, i, w_dt);
+        }
     }
-}
+    // this lane's sum of squares
+    __device__ __forceinline__ float squares(const void* x, int x_dt, int64_t base, int64_t d, int t, int stride) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            const int64_t i = t + (int64_t)e * stride;
+            v[e] = i < d ? word_to_f32(xw[e], x, base + i, x_dt) : 0.0f;
+            ss = fmaf(v[e], v[e], ss);
+        }
+        return ss;
+    }
+    __device__ __forceinline__ void store(void* out, int out_dt, int64_t base, const void* w, int w_dt, int64_t d, int t,
+                                          int stride, float inv) {
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            const int64_t i = t + (int64_t)e * stride;
+            if (i < d) st_act(out, base + i, (v[e] * inv) * word_to_f32(ww[e], w, i, w_dt), out_dt);
+        }
+    }
+};
 
 template <int PER>
 __global__ __launch_bounds__(256) void rms_norm_wave_kernel(const void* __restrict__ x, int x_dt,
@@ -115,18 +141,11 @@ __global__ __launch_bounds__(256) void rms_norm_wave_kernel(const void* __restri
     const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (r >= rows) return;
-    float v[PER];
-    load_row<PER>(x, x_dt, r * d, d, lane, 64, v);
-    float ss = 0.0f;
-#pragma unroll
-    for (int e = 0; e < PER; e++) ss = fmaf(v[e], v[e], ss);
-    ss = wave_sum(ss);
+    NormRow<PER> n;
+    n.load(x, x_dt, r * d, w, w_dt, d, lane, 64);
+    const float ss = wave_sum(n.squares(x, x_dt, r * d, d, lane, 64));
     const float inv = 1.0f / (float)sqrt((double)(ss / (float)d + eps));
-#pragma unroll
-    for (int e = 0; e < PER; e++) {
-        const int64_t i = lane + (int64_t)e * 64;
-        if (i < d) st_act(out, r * d + i, (v[e] * inv) * ld_act(w, i, w_dt), out_dt);
-    }
+    n.store(out, out_dt, r * d, w, w_dt, d, lane, 64, inv);
 }
 
 template <int PER>
@@ -135,18 +154,11 @@ __global__ __launch_bounds__(256) void rms_norm_block_kernel(const void* __restr
                                                              void* __restrict__ out, int out_dt, int64_t d) {
     __shared__ float red[4];
     const int64_t r = blockIdx.x;
-    float v[PER];
-    load_row<PER>(x, x_dt, r * d, d, threadIdx.x, 256, v);
-    float ss = 0.0f;
-#pragma unroll
-    for (int e = 0; e < PER; e++) ss = fmaf(v[e], v[e], ss);
-    ss = block_sum256(ss, red);
+    NormRow<PER> n;
+    n.load(x, x_dt, r * d, w, w_dt, d, threadIdx.x, 256);
+    const float ss = block_sum256(n.squares(x, x_dt, r * d, d, threadIdx.x, 256), red);
     const float inv = 1.0f / (float)sqrt((double)(ss / (float)d + eps));
-#pragma unroll
-    for (int e = 0; e < PER; e++) {
-        const int64_t i = threadIdx.x + (int64_t)e * 256;
-        if (i < d) st_act(out, r * d + i, (v[e] * inv) * ld_act(w, i, w_dt), out_dt);
-    }
+    n.store(out, out_dt, r * d, w, w_dt, d, threadIdx.x, 256, inv);
 }
 
 // Rows longer than 256 * 64 elements: two passes over x.
@@ -166,32 +178,54 @@ __global__ __launch_bounds__(256) void rms_norm_long_kernel(const void* __restri
         st_act(out, r * d + i, (ld_act(x, r * d + i, x_dt) * inv) * ld_act(w, i, w_dt), out_dt);
 }
 
-// ---- RoPE: one thread per rotated pair --------------------------------------------
+// ---- RoPE: one thread per rotated pair and position --------------------------------
+// The rows at one position (row % L) of a group of `per` heads share a pair's
+// factors: a thread evaluates pow, cos and sin once (in double, as the CPU backend
+// does) and rotates that pair of its group's rows. Bound: the factors and the memory
+// round trips of a thread's rows: 1500 positions of 32 and of 8 heads of 128 take
+// 16.8 us a launch on average on MI355X, 30.8 with the factors evaluated per row.
 __global__ __launch_bounds__(256) void rope_kernel(const void* __restrict__ x, int x_dt, void* __restrict__ out,
                                                    int out_dt, int64_t rows, int64_t L, int64_t D, int dims,
                                                    int traditional, float base, float scale, int64_t offset,
-                                                   const float* __restrict__ freqs) {
+                                                   const float* __restrict__ freqs, int64_t per) {
     const int half = dims / 2;
     const int64_t per_row = D - half;  // pairs plus pass-through features
-    const int64_t total = rows * per_row;
+    const int64_t heads = (rows + L - 1) / L, groups = (heads + per - 1) / per;
+    const int64_t total = groups * L * per_row;
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = t / per_row;
-        const int i = (int)(t - r * per_row);
-        const int64_t o = r * D;
+        const int64_t gl = t / per_row;
+        const int i = (int)(t - gl * per_row);
+        const int64_t g = gl / L, l = gl - g * L;
+        const int64_t h0 = g * per, h1 = min(heads, h0 + per);
         if (i >= half) {  // features past `dims` pass through
             const int64_t f = dims + (i - half);
-            if (f < D) st_act(out, o + f, ld_act(x, o + f, x_dt), out_dt);
+            for (int64_t h = h0; h < h1; h++) {
+                const int64_t o = (h * L + l) * D;
+                if (f < D && h * L + l < rows) st_act(out, o + f, ld_act(x, o + f, x_dt), out_dt);
+            }
             continue;
         }
         const float inv = freqs ? 1.0f / freqs[i] : (float)pow((double)base, -(double)(2 * i) / (double)dims);
-        const float pos = (float)(offset + r % L);
+        const float pos = (float)(offset + l);
         const float theta = pos * scale * inv;
         const float c = (float)cos((double)theta), s = (float)sin((double)theta);
-        const int64_t i0 = traditional ? o + 2 * i : o + i;
-        const int64_t i1 = traditional ? o + 2 * i + 1 : o + i + half;
-        const float a = ld_act(x, i0, x_dt), b = ld_act(x, i1, x_dt);
-        st_act(out, i0, a * c - b * s, out_dt);
-        st_act(out, i1, a * s + b * c, out_dt);
+        const int64_t j0 = traditional ? 2 * i : i, j1 = traditional ? 2 * i + 1 : i + half;
+        for (int64_t h = h0; h < h1; h += 4) {  // four rows' loads together
+            uint32_t aw[4], bw[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int64_t o = min((min(h + q, h1 - 1) * L + l), rows - 1) * D;
+                aw[q] = ld_word(x, o + j0, x_dt), bw[q] = ld_word(x, o + j1, x_dt);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int64_t r = (h + q) * L + l;
+                if (h + q >= h1 || r >= rows) break;
+                const float a = word_to_f32(aw[q], x, r * D + j0, x_dt), b = word_to_f32(bw[q], x, r * D + j1, x_dt);
+                st_act(out, r * D + j0, a * c - b * s, out_dt);
+                st_act(out, r * D + j1, a * s + b * c, out_dt);
+            }
+        }
     }
 }
 
@@ -1540,10 +1574,15 @@ Status launch_rms_norm(const void* x, int x_dt, const void* w, int w_dt, float e
 
 Status launch_rope(const void* x, int x_dt, void* out, int out_dt, int64_t rows, int64_t L, int64_t D, int dims,
                    bool traditional, float base, float scale, int64_t offset, const float* freqs, hipStream_t st) {
-    const int64_t total = rows * (D - dims / 2);
-    if (total == 0) return Status::ok();
-    hipLaunchKernelGGL(rope_kernel, dim3(grid_for(total, 256, 16384)), dim3(256), 0, st, x, x_dt, out, out_dt, rows,
-                       L, D, dims, traditional ? 1 : 0, base, scale, offset, freqs);
+    if (rows == 0) return Status::ok();
+    L = std::min(L, rows);  // (the position of a row is row % L)
+    const int64_t heads = (rows + L - 1) / L, pairs = L * (D - dims / 2);
+    if (heads * pairs == 0) return Status::ok();
+    // heads per thread: as many as leave four blocks of threads per CU (the factors
+    // are evaluated once per thread; with few positions, one head per thread)
+    const int64_t per = std::max<int64_t>(1, std::min<int64_t>(heads, heads * pairs / (4 * 256 * 256)));
+    hipLaunchKernelGGL(rope_kernel, dim3(grid_for((heads + per - 1) / per * pairs, 256, 16384)), dim3(256), 0, st, x, x_dt,
+                       out, out_dt, rows, L, D, dims, traditional ? 1 : 0, base, scale, offset, freqs, per);
     return Status::ok();
 }
 

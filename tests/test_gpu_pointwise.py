@@ -103,3 +103,40 @@ def test_copy_broadcast_and_reverse(hip):
     want = np.full((2, 3, 40), -1, np.float32)
     want[:, :, :16] = a[3:0:-1]
     np.testing.assert_array_equal(hip.Floats(out), want)
+
+
+@pytest.mark.parametrize("heads,L,D,dims,traditional", [(1, 1, 128, 128, False), (40, 700, 128, 128, False),
+                                                        (33, 300, 96, 64, False), (6, 301, 64, 64, True),
+                                                        (130, 70, 128, 32, False)])
+@pytest.mark.parametrize("dt", [F32, BF16])
+def test_rope_head_groups(hip, oracle, heads, L, D, dims, traditional, dt):
+    """Heads that share a position's factors, in whole groups and not."""
+    rng = np.random.default_rng(heads + L)
+    raw, x = _bits(rng.standard_normal((1, heads, L, D)), dt)
+    t = hip.FromRaw(dt, raw, *raw.shape)
+    step(f"jh_rope heads={heads} L={L} D={D} dims={dims} {dt}")
+    got = hip.Floats(hip.RoPE(t, dims, traditional, 1e6, 1.0, 17, out_dtype=F32))
+    want = oracle.rope(x, dims, traditional, 1e6, 1.0, 17)
+    assert np.abs(got - want).max() <= 1e-6 * np.abs(want).max()  # two products and a sum: 3 * 2^-24, and a rounded angle
+    # a call of fewer rows than positions, and one that ends inside a head
+    for rows, Lc in ((3, 1000), (L + L // 2, L)):
+        if rows <= heads * L:
+            out = hip.FromFloats(np.zeros((rows, D), np.float32))
+            _lib.check(hip._ctx, hip._L.jh_rope(hip._ctx, t.ptr, dt, rows, Lc, D, dims, int(traditional), 1e6, 1.0, 17, None,
+                                                out.ptr, F32))
+            np.testing.assert_array_equal(hip.Floats(out), got.reshape(-1, D)[:rows])
+
+
+@pytest.mark.parametrize("rows,d", [(3, 1), (5, 63), (2, 129), (9, 1024), (2, 1025), (3, 4095), (1, 12288), (2, 16385)])
+@pytest.mark.parametrize("x_dt,w_dt", [(F32, BF16), (BF16, F16), (BF16, F32)])
+def test_rms_norm_lengths(hip, oracle, rows, d, x_dt, w_dt):
+    """Row lengths at the ends of each kernel's range, odd ones among them."""
+    rng = np.random.default_rng(rows * d)
+    rx, x = _bits(rng.standard_normal((rows, d)), x_dt)
+    rw, w = _bits(1 + 0.1 * rng.standard_normal(d), w_dt)
+    step(f"jh_rms_norm rows={rows} d={d} x={x_dt} w={w_dt}")
+    got = hip.Floats(hip.RMSNorm(hip.FromRaw(x_dt, rx, rows, d), hip.FromRaw(w_dt, rw, d), 1e-6, out_dtype=F32))
+    want = oracle.rms_norm(x, w, 1e-6)
+    # the oracle adds the d squares one after another, each sum rounded: up to
+    # d * 2^-24 of it, half that in its root (the kernel adds at most 65 in a row)
+    assert np.abs(got - want).max() <= (2.0 ** -22 + 0.5 * d * 2.0 ** -24) * np.abs(want).max()
