@@ -72,19 +72,21 @@ __device__ __forceinline__ float widen_sb(uint32_t bits) {
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
 // One packed word -> 8 bf16 weights fl32(q*s + b) rounded to nearest even, in
-// word order (q0 = lowest nibble): 3 masks, 8 v_cvt_f32_ubyteN, 8 FMAs and 4
-// v_cvt_pk_bf16_f32.
+// word order (q0 = lowest nibble): 3 masks, 4 conversions, 8 FMAs and 4
+// v_cvt_pk_bf16_f32. A byte holding a 4-bit code q, read as e4m3, is q * 2^-9
+// (subnormal or not), so v_cvt_scalef32_pk_f32_fp8 with scale 512 gives two codes
+// as fp32 exactly.
 __device__ __forceinline__ bf16x8_t dequant_word(uint32_t word, float sc, float bi) {
-    uint32_t lo = word & 0x0F0F0F0Fu, hi = (word >> 4) & 0x0F0F0F0Fu;
-    // An empty asm hides where lo and hi came from, so the byte extractions
-    // below stay single v_cvt_f32_ubyteN instead of being re-derived as
-    // per-nibble shifts and masks of `word`.
-    asm("" : "+v"(lo), "+v"(hi));
+    const uint32_t lo = word & 0x0F0F0F0Fu, hi = (word >> 4) & 0x0F0F0F0Fu;
+    const f32x2_t e0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.0f, false);  // q0 q2
+    const f32x2_t e1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.0f, true);   // q4 q6
+    const f32x2_t o0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.0f, false);  // q1 q3
+    const f32x2_t o1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.0f, true);   // q5 q7
+    const float q[8] = {e0.x, o0.x, e0.y, o0.y, e1.x, o1.x, e1.y, o1.y};
     uint32_t o[4];
 #pragma unroll
     for (int p = 0; p < 4; p++) {
-        const f32x2_t f = {fmaf((float)((lo >> (8 * p)) & 0xFFu), sc, bi),
-                           fmaf((float)((hi >> (8 * p)) & 0xFFu), sc, bi)};
+        const f32x2_t f = {fmaf(q[2 * p], sc, bi), fmaf(q[2 * p + 1], sc, bi)};
         o[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_t));
     }
     return __builtin_bit_cast(bf16x8_t, make_uint4(o[0], o[1], o[2], o[3]));
