@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import math
 
 import numpy as np
 
@@ -31,8 +32,9 @@ def _dense_strides(shape) -> tuple:
     st, acc = [], 1
     for d in reversed(shape):
         st.append(acc)
-        acc *= int(d)
-    return tuple(reversed(st))
+        acc *= d
+    st.reverse()
+    return tuple(st)
 
 
 class Tensor:
@@ -44,26 +46,30 @@ class Tensor:
                  strides=None):
         self._b = backend
         self.ptr = int(ptr) if ptr else 0
-        self.shape = tuple(int(d) for d in shape)
+        self.shape = shape = tuple(map(int, shape))
         self.dtype = dtype
         self._owned = owned
         self._keep = keep  # an object whose lifetime covers the memory (non-owned views)
-        self.strides = tuple(int(x) for x in strides) if strides is not None else _dense_strides(self.shape)
+        self.strides = tuple(map(int, strides)) if strides is not None else _dense_strides(shape)
         if backend is not None and owned and backend._sweeper is not None:
             backend._sweeper.track(self)
 
     @property
     def contiguous(self) -> bool:
         """Row-major dense (strides of length-1 axes do not matter)."""
-        dense = _dense_strides(self.shape)
-        return all(n == 1 or a == b for n, a, b in zip(self.shape, self.strides, dense))
+        acc = 1
+        for n, st in zip(reversed(self.shape), reversed(self.strides)):
+            if n != 1 and st != acc:
+                return False
+            acc *= n
+        return True
 
     def Shape(self) -> list:
         return list(self.shape)
 
     @property
     def numel(self) -> int:
-        return int(np.prod(self.shape, dtype=np.int64)) if self.shape else 1
+        return math.prod(self.shape)
 
     @property
     def nbytes(self) -> int:
@@ -79,7 +85,8 @@ class Tensor:
         self.ptr = 0
 
     def __del__(self):
-        self.free()
+        if getattr(self, "_owned", False):
+            self.free()
 
     def __repr__(self):
         return f"Tensor({DTYPE_NAME[self.dtype]}, {list(self.shape)})"
@@ -282,7 +289,7 @@ class HipBackend:
             self._arena = prev
 
     def empty(self, dtype: int, *shape) -> Tensor:
-        n = int(np.prod(shape, dtype=np.int64)) if shape else 1
+        n = math.prod(map(int, shape))
         if self._arena is not None:
             base, off = self._arena
             need = max(1, n * DTYPE_SIZE[dtype])
@@ -365,7 +372,7 @@ class HipBackend:
         """The result buffer of an operator: `out` when given (checked: dense,
         exactly the result's element count, a dtype the operator writes and, when
         out_dtype is also given, that dtype), else a new tensor of `shape`."""
-        n = int(np.prod(shape, dtype=np.int64)) if len(shape) else 1
+        n = math.prod(shape)
         if out is None:
             dt = out_dtype if out_dtype is not None else default_dtype
             if dt not in dtypes:
@@ -439,7 +446,7 @@ class HipBackend:
         k = P * (32 // bits)
         rs = rhsIndices.shape
         K = rs[-1]
-        n_lead = int(np.prod(rs[:-1], dtype=np.int64)) if len(rs) > 1 else 1
+        n_lead = math.prod(rs[:-1]) if len(rs) > 1 else 1
         # transpose=false: each slot's MatMul(x, Dequantize(W_e)), x features = n
         x_feat, y_feat = (k, n) if transpose else (n, k)
         if x.shape[-1] != x_feat or len(x.shape) < 3:
@@ -494,9 +501,9 @@ class HipBackend:
         -1 allowed), else of a dense copy."""
         shape = list(shape)
         if shape.count(-1) == 1:
-            known = int(np.prod([d for d in shape if d != -1], dtype=np.int64))
+            known = math.prod([d for d in shape if d != -1])
             shape[shape.index(-1)] = x.numel // known if known else 0
-        if int(np.prod(shape, dtype=np.int64)) != x.numel:
+        if math.prod(shape) != x.numel:
             raise JanisHipError(_lib.JH_ERR_INVALID, f"Reshape: {list(x.shape)} -> {shape}")
         x = self._c(x)
         return Tensor(self, x.ptr, shape, x.dtype, owned=False, keep=x)
@@ -675,8 +682,8 @@ class HipBackend:
     @staticmethod
     def _axis_view(x: Tensor, axis: int) -> tuple:
         axis = axis % len(x.shape)
-        outer = int(np.prod(x.shape[:axis], dtype=np.int64))
-        inner = int(np.prod(x.shape[axis + 1:], dtype=np.int64))
+        outer = math.prod(x.shape[:axis])
+        inner = math.prod(x.shape[axis + 1:])
         return axis, outer, x.shape[axis], inner
 
     def Softmax(self, x: Tensor, axis: int) -> Tensor:
@@ -1022,7 +1029,7 @@ class HipBackend:
             raise JanisHipError(_lib.JH_ERR_INVALID, "MoeSwiGLU: stack shapes do not match")
         rs = rhsIndices.shape
         K = rs[-1]
-        n_tok = int(np.prod(rs[:-1], dtype=np.int64)) if len(rs) > 1 else 1
+        n_tok = math.prod(rs[:-1]) if len(rs) > 1 else 1
         if x.shape[-1] != H or x.numel != n_tok * H:
             raise JanisHipError(_lib.JH_ERR_INVALID, f"MoeSwiGLU: x {list(x.shape)} vs hidden={H}")
         y = self._result("MoeSwiGLU", out, out_dtype, F32, (*rs[:-1], H))
