@@ -140,11 +140,28 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
     float c = fabsf(a.scale) * kLog2e;  // the scale's sign goes into q
     {
         const float sgn = a.scale < 0.0f ? -1.0f : 1.0f;
-        float qscale = sgn, amax = 0.0f;
+        float qscale = sgn, amax = 0.0f, v[8][8];
+#pragma unroll
+        for (int kk = 0; kk < 8; kk++) {
+            const int64_t at = q_off + 16 * kk + 8 * h;
+            if (a.q_dt == JH_F32) {
+                const float4* const p = reinterpret_cast<const float4*>(static_cast<const float*>(a.q) + at);
+                const float4 x = p[0], y = p[1];
+                v[kk][0] = x.x, v[kk][1] = x.y, v[kk][2] = x.z, v[kk][3] = x.w;
+                v[kk][4] = y.x, v[kk][5] = y.y, v[kk][6] = y.z, v[kk][7] = y.w;
+            } else {
+                const uint4 x = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.q) + at);
+                const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                for (int p = 0; p < 4; p++)
+                    v[kk][2 * p] = __uint_as_float(w[p] << 16), v[kk][2 * p + 1] = __uint_as_float(w[p] & 0xFFFF0000u);
+            }
+        }
         if constexpr (F16) {
+#pragma unroll
             for (int kk = 0; kk < 8; kk++)
 #pragma unroll
-                for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(load_act(a.q, q_off + 16 * kk + 8 * h + e, a.q_dt)));
+                for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[kk][e]));
             amax = pair32<true>(amax);
             const int ex = (int)(__float_as_uint(amax) >> 23);
             const int f = min(max(267 - ex, 1), 253);  // exponent field of 2^(13 - exponent of amax)
@@ -153,12 +170,10 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
         }
 #pragma unroll
         for (int kk = 0; kk < 8; kk++) {
-            float v[8];
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = load_act(a.q, q_off + 16 * kk + 8 * h + e, a.q_dt) * qscale;
             uint32_t t[4][QN];
 #pragma unroll
-            for (int p = 0; p < 4; p++) split_pair<F16, QN>(v[2 * p], v[2 * p + 1], t[p]);
+            for (int p = 0; p < 4; p++)
+                split_pair<F16, QN>(v[kk][2 * p] * qscale, v[kk][2 * p + 1] * qscale, t[p]);
 #pragma unroll
             for (int n = 0; n < QN; n++) qf[n][kk] = make_uint4(t[0][n], t[1][n], t[2][n], t[3][n]);
         }
@@ -368,7 +383,10 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
     }
 }
 
-// The splits of one row added in split order (one wave per row).
+// The splits of one row added in split order: one wave per row, lane s holding
+// split s's maximum and sum (at most 64 splits), the values requested 8 splits at
+// a time, so that a row costs three memory round trips up to 16 splits.
+constexpr int kMaxSplits = 64;
 __global__ __launch_bounds__(256) void sdpa_mfma_merge_kernel(const float* __restrict__ part_o,
                                                               const float* __restrict__ part_ml, int64_t rows,
                                                               int n_rows, int G, int Lq, int nsplit,
@@ -378,18 +396,24 @@ __global__ __launch_bounds__(256) void sdpa_mfma_merge_kernel(const float* __res
     if (row >= rows) return;
     const int64_t bhk = row / n_rows;
     const int r = (int)(row - bhk * n_rows);
-    const float* const ml = part_ml + row * nsplit * 2;
-    float mx = -__builtin_inff();
-    for (int s = 0; s < nsplit; s++) mx = fmaxf(mx, ml[2 * s]);
-    float l = 0.0f, x0 = 0.0f, x1 = 0.0f;
-    for (int s = 0; s < nsplit; s++) {
-        const float m = ml[2 * s];
-        if (m == -__builtin_inff() && ml[2 * s + 1] == 0.0f) continue;  // no keys of the row in this split
-        const float w = m == mx ? 1.0f : __builtin_amdgcn_exp2f(m - mx);
-        const float2 o = *reinterpret_cast<const float2*>(part_o + (row * nsplit + s) * kDh + 2 * lane);
-        l = fmaf(ml[2 * s + 1], w, l);
-        x0 = fmaf(o.x, w, x0);
-        x1 = fmaf(o.y, w, x1);
+    const float2 ml = reinterpret_cast<const float2*>(part_ml)[row * nsplit + min(lane, nsplit - 1)];
+    const float mx = wave_max(ml.x);
+    // (a split without keys of the row: a sum of 0 and values of 0)
+    const float w = lane >= nsplit ? 0.0f : ml.x == mx ? 1.0f : __builtin_amdgcn_exp2f(ml.x - mx);
+    const float l = wave_sum(lane >= nsplit ? 0.0f : ml.y * w);
+    float x0 = 0.0f, x1 = 0.0f;
+    for (int s0 = 0; s0 < nsplit; s0 += 8) {
+        float2 o[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            o[j] = *reinterpret_cast<const float2*>(part_o + (row * nsplit + min(s0 + j, nsplit - 1)) * kDh + 2 * lane);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if (s0 + j >= nsplit) break;
+            const float ws = __shfl(w, s0 + j, 64);
+            x0 = fmaf(o[j].x, ws, x0);
+            x1 = fmaf(o[j].y, ws, x1);
+        }
     }
     const int64_t at = ((bhk * G + r % G) * Lq + r / G) * kDh + 2 * lane;
     store_y(out, at, x0 / l, out_dt);
@@ -411,11 +435,23 @@ bool sdpa_mfma_ok(const void* q, int q_dt, const void* k, const void* v, int kv_
            aligned16(v) && aligned16(out);
 }
 
-// Splits of the keys: one while the row tiles fill the GPU (two blocks per CU);
-// fewer tiles take enough splits to fill it, at least 256 keys each.
+// Splits of the keys: the count with the least modelled time. On MI355X a 64-key
+// tile of 128 rows took 2.4 us in a block alone on its CU and 3.1 us in each of two
+// that share one, the merge 4 us and its partials (written and read at about 4
+// TB/s). 512 queries of 512 keys stay whole (27 us; in halves 31), 1500 of 4000 too
+// (197; in halves 205), 16 of 4112 take 22 splits (23.5 us; 28.6 with 16 and a merge
+// of one split at a time).
 int64_t sdpa_mfma_splits(int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int num_cus) {
-    const int64_t blocks = B * Hk * ((Hq / Hk * Lq + kRows - 1) / kRows);
-    return std::max<int64_t>(1, std::min<int64_t>(2 * (int64_t)num_cus / blocks, Lk / 256));
+    const int64_t blocks = B * Hk * ((Hq / Hk * Lq + kRows - 1) / kRows), tiles = (Lk + kKeys - 1) / kKeys;
+    int64_t best = 1;
+    double least = 0;
+    for (int64_t n = 1; n <= tiles && n <= kMaxSplits; n++) {
+        const int64_t per_cu = (blocks * n + num_cus - 1) / num_cus;
+        const double work = (3.1 * (double)(per_cu / 2) + 2.4 * (double)(per_cu % 2)) * (double)((tiles + n - 1) / n);
+        const double t = work + (n > 1 ? 4.0 + (double)(B * Hq * Lq * n) * (2 * (kDh + 2) * 4) / 4e6 : 0.0);
+        if (n == 1 || t < least) best = n, least = t;
+    }
+    return best;
 }
 
 size_t sdpa_mfma_workspace_bytes(int64_t B, int64_t Hq, int64_t Lq, int64_t nsplit) {
