@@ -122,3 +122,24 @@ def test_moe_route_sizes(hip, oracle, E, k):
     # a NaN or an infinity makes every probability NaN: nothing is larger than
     # the first, so the order stays
     assert np.array_equal(got_i[6:], np.tile(np.arange(k, dtype=np.int32), (2, 1))) and np.isnan(got_s[6:]).all()
+
+
+@pytest.mark.parametrize("gs", [64, 128])
+def test_gather_scales_at_two_bytes(hip, oracle, gs):
+    """Scales and biases that start at an odd element (2-byte aligned) keep
+    their results: such calls stay on the dot products."""
+    E, n, k = 2, 64, 512
+    idx = _buckets((40, 24), 4, 5)
+    q = synth.quant_linear(850, n, k, gs, lead=(E,))
+    w = upload_quant(hip, q)[0]
+    shifted = []
+    for bits in (q.s_bits, q.b_bits):
+        flat = hip.FromBF16Bits(np.concatenate([np.zeros(1, np.uint16), np.asarray(bits, np.uint16).ravel()]),
+                                bits.size + 1)
+        shifted.append(hip.Wrap(flat.ptr + 2, bits.shape, BF16, keep=flat))
+    xb, x = synth.activations(851, (16, 4, 1, k))
+    step(f"jh_gather_quant_matmul, scales 2-byte aligned, gs={gs}")
+    y = hip.Floats(hip.GatherQuantMatmul(hip.FromBF16Bits(xb, 16, 4, 1, k), w, *shifted, hip.FromInt32(idx), True, gs, 4,
+                                         out_dtype=F32))
+    ok, d, sc = rel_ok(y, oracle.gather_quant_matmul(x, q.w, q.s, q.b, idx, gs), 1e-5)
+    assert ok, (d, sc)
