@@ -1866,10 +1866,20 @@ Status launch_rope_table(int dims, float base, float scale, int64_t pos, const f
     return Status::ok();
 }
 
+// In pieces of 8 from this many elements, below one by one: with fewer the chip is
+// not full and a thread's eight elements (for SiLU its eight exponentials) come one
+// after the other. bf16 on MI355X, one by one / in pieces: Add of 12288 elements
+// 2.4 / 3.0 us, 400000 3.1 / 3.1, 800000 3.9 / 3.4, 2^22 11.8 / 6.1; SiLU(a) * b of
+// 98304 3.1 / 4.6, 786432 5.5 / 5.1, 1228800 6.2 / 6.0, 2^22 13.2 / 9.8 (SiLU one by
+// one measured with the library's exponential).
+constexpr int64_t kAddVecMin = (int64_t)1 << 19, kSiluVecMin = (int64_t)1 << 20;
+
 Status launch_elementwise(int op, const void* a, int a_dt, const void* b, int b_dt, void* out, int out_dt, int64_t n,
                           hipStream_t st) {
     if (n == 0) return Status::ok();
-    const bool vec = aligned16(a) && aligned16(out) && (op == JH_OP_SILU || aligned16(b));
+    const bool silu = op == JH_OP_SILU || op == JH_OP_SILU_MUL;
+    const bool vec = aligned16(a) && aligned16(out) && (op == JH_OP_SILU || aligned16(b)) &&
+                     n >= (silu ? kSiluVecMin : kAddVecMin);
     auto go = [&](auto kern, int64_t per) {
         hipLaunchKernelGGL(kern, dim3(grid_for(n, 256 * per, 16384)), dim3(256), 0, st, op, a, a_dt, b, b_dt, out, out_dt, n);
     };
