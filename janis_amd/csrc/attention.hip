@@ -11,15 +11,23 @@
 // operand where they are, with no exchange between lanes (its K order is the
 // order the first product left the keys in, applied to V as it is staged).
 //
-// Precision is that of fp32 arithmetic. Keys and values enter as they are
-// stored. Queries and probabilities are fp32 and enter as sums of 16-bit terms,
-// one matrix instruction per term into the same fp32 accumulator:
+// Keys and values enter as they are stored. Queries and probabilities are fp32
+// and enter as sums of 16-bit terms, one matrix instruction per term into the
+// same fp32 accumulator:
 //   f16 keys:  a row of q times a power of two that brings its largest element
 //              to [2^13, 2^14) (its inverse joins the softmax scale), as one f16
-//              term for bf16 q (exact) and two for fp32 q (22 bits and a sign);
-//              p * 2^7 as two f16 terms;
+//              term for bf16 q (exact for elements down to 2^-30 of the largest)
+//              and two for fp32 q (within 2^-24 of the element, or 2^-38 of the
+//              largest where that is more);
+//              p * 2^13, at most 2^15, as two f16 terms: within 2^-24 of p or, f16
+//              having nothing below 2^-24, 2^-38 of the row's maximum, 1;
 //   bf16 keys: one bf16 term for bf16 q, three for fp32 q (24 bits); p as three
 //              bf16 terms.
+// The floor under f16 probabilities shows only where the keys that hold the weight
+// have next to no values (an attention sink), so that the result comes from the
+// small ones. Each row's result is held against it, by the sum of the squares of the
+// block's values (3 % of a call's time), and a row that it could have cost more than
+// about 2^-22 is computed again as rows that are not finite are.
 // Relative error against float64 with scores of standard deviation 2.3, 512 and
 // 4000 keys: 3.9e-7 and 7.9e-7 (fp32 q, f16 keys), where the per-row kernel
 // (sdpa_rows_kernel) has 7.3e-7 and 1.5e-6; with bf16 q and keys 2.8e-7 and
@@ -47,8 +55,8 @@ constexpr int kRows = 128;  // rows per block
 constexpr int kKeys = 64;   // keys per tile
 constexpr int kTileBytes = kKeys * kDh * 2;
 constexpr float kLog2e = 1.44269504088896340736f;
-constexpr float kPShift = 7.0f;   // p is held as p * 2^7
-constexpr float kLazy = 8.0f;     // a row's maximum is moved when it grew by more than this (log2)
+constexpr float kPShift = 13.0f;  // p is held as p * 2^13
+constexpr float kLazy = 2.0f;     // a row's maximum is moved when it grew by more than this (log2)
 
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
@@ -193,6 +201,7 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
     const auto rv = make_rsrc(a.v + head, (uint32_t)a.Lk * kDh * 2);
     const int sr = tid >> 4, sc = tid & 15;  // staging: row and 16-byte chunk
     u32x4_t kr[4], vr[4];
+    float v2 = 0.0f;  // F16: sum of the squares of the values this thread stages
     auto load = [&](int k0) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -206,6 +215,14 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
             const int k = sr + 16 * j;
             *reinterpret_cast<u32x4_t*>(buf + k * 256 + 16 * (sc ^ (k & 15))) = kr[j];
         }
+        if constexpr (F16)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const f16x2_t v = __builtin_bit_cast(f16x2_t, (uint32_t)vr[j][d]);
+                    v2 = __builtin_amdgcn_fdot2(v, v, v2, false);
+                }
         uint8_t* const vt = buf + kTileBytes;
 #pragma unroll
         for (int d = 0; d < 4; d++) {
@@ -265,20 +282,23 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
                 ls += s[g][r];
             }
         l += ls;
+        // B of step kk: keys 16 kk + 4 h + 0..3, then 16 kk + 8 + 4 h + 0..3
         const uint8_t* const vt = buf + kTileBytes;
+        auto value_frag = [&](int kk, int d) {
+            const int f = 32 * d + c32, x = (f >> 1) & 15;
+            const uint2 lo = *reinterpret_cast<const uint2*>(vt + f * 128 + 8 * ((4 * kk + h) ^ x));
+            const uint2 hi = *reinterpret_cast<const uint2*>(vt + f * 128 + 8 * ((4 * kk + 2 + h) ^ x));
+            return make_uint4(lo.x, lo.y, hi.x, hi.y);
+        };
 #pragma unroll
         for (int kk = 0; kk < 4; kk++) {
-            // B: keys 16 kk + 4 h + 0..3, then 16 kk + 8 + 4 h + 0..3
-            const int g = kk >> 1, r0 = 8 * (kk & 1);
             uint32_t t[4][PN];
 #pragma unroll
-            for (int p = 0; p < 4; p++) split_pair<F16, PN>(s[g][r0 + 2 * p], s[g][r0 + 2 * p + 1], t[p]);
+            for (int p = 0; p < 4; p++)
+                split_pair<F16, PN>(s[kk >> 1][8 * (kk & 1) + 2 * p], s[kk >> 1][8 * (kk & 1) + 2 * p + 1], t[p]);
 #pragma unroll
             for (int d = 0; d < 4; d++) {
-                const int f = 32 * d + c32, x = (f >> 1) & 15;
-                const uint2 lo = *reinterpret_cast<const uint2*>(vt + f * 128 + 8 * ((4 * kk + h) ^ x));
-                const uint2 hi = *reinterpret_cast<const uint2*>(vt + f * 128 + 8 * ((4 * kk + 2 + h) ^ x));
-                const uint4 vf = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                const uint4 vf = value_frag(kk, d);
 #pragma unroll
                 for (int n = PN - 1; n >= 0; n--)
                     o[d] = mfma<F16>(vf, make_uint4(t[0][n], t[1][n], t[2][n], t[3][n]), o[d]);
@@ -308,6 +328,23 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int r = 0; r < 16; r++) bad |= !finite(o[t][r]);
+    if constexpr (F16) {
+        // p * 2^13 is off by up to 2^-25 where it is small, so the result by about
+        // 2^-25 / sqrt(3) of the root of the sum of V^2: under 2^-22 of the result
+        // unless that is as small as here. (An infinity in V counts as the largest
+        // sum of finite values.)
+        __shared__ float v2s[4];
+        v2 = wave_sum(v2);
+        if (lane == 0) v2s[wave] = v2;
+        __syncthreads();
+        const float all = fminf((v2s[0] + v2s[1]) + (v2s[2] + v2s[3]), 0x1p39f * (float)(ke_all - kb));
+        float o2 = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) o2 = fmaf(o[t][r], o[t][r], o2);
+        bad |= l > 0.0f && pair32<false>(o2) < 0x1p-7f * all;
+    }
     const uint64_t votes = __ballot(bad && w0 + c32 < n_rows);
     uint32_t again = (uint32_t)votes | (uint32_t)(votes >> 32);  // rows of the wave to compute again
     const int64_t grow = (int64_t)bhk * n_rows;

@@ -121,3 +121,30 @@ def test_sdpa_mfma_captured_without_workspace(oracle):
         ok, dd, sc = rel_ok(b.Floats(out[-1]), want, 1e-5)
         assert ok, (dd, sc)
     b.Close()
+
+
+@pytest.mark.parametrize("kv_dt", [F16, BF16])
+@pytest.mark.parametrize("Lk", [200, 700])
+@pytest.mark.parametrize("gap", [6, 12, 16, 20, 30, 45])
+def test_sdpa_mfma_dominant_key(hip, gap, Lk, kv_dt):
+    """One key holds all but 2^-gap of a row's weight and its values are zero (an
+    attention sink): the result is the sum over the small probabilities, which
+    keep fp32's relative precision. A score of gap * ln 2 nats and its difference
+    to the maximum are rounded to fp32 (the dominant score is exact, the others
+    are below 2): 2^-24 of gap each way of writing it, three roundings, and the
+    exponential's and the sums' own 2^-22."""
+    Lq = 40
+    q, k, v = _case(1, 2, 1, Lq, Lk, F32, kv_dt, spread=0.2)
+    at = Lk // 3
+    q[..., 0] = 1.0
+    k[..., 0] = 0.0
+    k[0, 0, at] = 0.0
+    k[0, 0, at, 0] = _round(np.float32([gap * np.log(2.0)]), kv_dt)[0]
+    v[0, 0, at] = 0.0
+    step(f"jh_sdpa rows, a dominant key, gap={gap} Lk={Lk} kv={kv_dt}")
+    got = hip.Floats(hip.SDPA(_put(hip, q, F32), _put(hip, k, kv_dt), _put(hip, v, kv_dt), 1.0, False)).astype(np.float64)
+    s = q[0].astype(np.float64) @ k[0, 0].astype(np.float64).T
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = (p @ v[0, 0].astype(np.float64)) / p.sum(-1, keepdims=True)
+    err = np.linalg.norm(got[0] - want, axis=-1) / np.linalg.norm(want, axis=-1)
+    assert err.max() <= 2.0 ** -22 + 3 * gap * 2.0 ** -24, err.max()
