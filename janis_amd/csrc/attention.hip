@@ -392,9 +392,12 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
         float mx = ninf;
         for (int key = kb + lane; key < lj; key += 64) mx = fmaxf(mx, score(key));
         mx = wave_max(mx);
+        // a split whose scores are all -inf adds nothing (and without splits the
+        // sum of 0 makes the row NaN)
+        const float sub = mx == ninf ? 0.0f : mx;
         float ls = 0.0f, x0 = 0.0f, x1 = 0.0f;
         for (int k0 = kb; k0 < lj; k0 += 64) {
-            const float e = k0 + lane < lj ? (float)exp((double)(score(k0 + lane) - mx)) : 0.0f;
+            const float e = k0 + lane < lj ? (float)exp((double)(score(k0 + lane) - sub)) : 0.0f;
             ls += e;
             for (int jj = 0; jj < min(64, lj - k0); jj++) {
                 const float p = __shfl(e, jj, 64);

@@ -148,3 +148,22 @@ def test_sdpa_mfma_dominant_key(hip, gap, Lk, kv_dt):
     want = (p @ v[0, 0].astype(np.float64)) / p.sum(-1, keepdims=True)
     err = np.linalg.norm(got[0] - want, axis=-1) / np.linalg.norm(want, axis=-1)
     assert err.max() <= 2.0 ** -22 + 3 * gap * 2.0 ** -24, err.max()
+
+
+@pytest.mark.parametrize("q_dt,kv_dt", [(F32, F16), (BF16, F16), (F32, BF16), (BF16, BF16)])
+@pytest.mark.parametrize("Lk,dead", [(100, 70), (700, 400)])
+def test_sdpa_mfma_scores_of_minus_infinity(hip, oracle, Lk, dead, q_dt, kv_dt):
+    """Keys whose scores are -inf have no weight, also where they fill whole key
+    tiles and whole splits; a row with no other key is NaN."""
+    q, k, v = _case(1, 4, 2, 20, Lk, q_dt, kv_dt)
+    q[..., 0] = 1.0
+    k[:, :, :dead, 0] = -np.inf
+    k[:, 1, :, 0] = -np.inf
+    step(f"jh_sdpa rows, scores of -inf, Lk={Lk} q={q_dt} kv={kv_dt}")
+    got = hip.Floats(hip.SDPA(_put(hip, q, q_dt), _put(hip, k, kv_dt), _put(hip, v, kv_dt), D ** -0.5, True, out_dtype=F32))
+    with np.errstate(all="ignore"):
+        want = oracle.sdpa(q, k, v, D ** -0.5, True)
+    assert np.isfinite(want[:, :2]).all() and np.isnan(want[:, 2:]).all()
+    assert np.isnan(got[:, 2:]).all()
+    ok, dd, sc = rel_ok(got[:, :2], want[:, :2], 1e-5)
+    assert ok, (dd, sc)
