@@ -35,8 +35,8 @@
 //
 // The products also meet keys past a row's limit with p = 0, where an infinity
 // or NaN in V would give NaN; the per-row kernel never reads those. So a row
-// whose result is not finite is computed again the way that kernel does (same
-// operations in the same order over the block's keys), and that result stands.
+// whose result is not finite is computed again with that kernel's arithmetic over
+// the block's keys, and that result stands.
 //
 // Bound: the matrix cores, with the softmax's VALU work beside them: per 32
 // rows x 64 keys, 16 MFMAs for each q term and 16 for each p term (512 cycles
@@ -54,6 +54,7 @@ constexpr int kDh = 128;
 constexpr int kRows = 128;  // rows per block
 constexpr int kKeys = 64;   // keys per tile
 constexpr int kTileBytes = kKeys * kDh * 2;
+constexpr int kAgain = 8;    // rows computed again together
 constexpr float kLog2e = 1.44269504088896340736f;
 constexpr float kPShift = 13.0f;  // p is held as p * 2^13
 constexpr float kLazy = 2.0f;     // a row's maximum is moved when it grew by more than this (log2)
@@ -375,51 +376,131 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
                 }
         }
     }
-    // rows with a result that is not finite: sdpa_rows_kernel's arithmetic over
-    // the block's keys, one row of the wave at a time
+    // Rows to compute again: sdpa_rows_kernel's arithmetic over the block's keys, kAgain
+    // rows of the wave together, so that they share each key's and value's loads (a
+    // lane scores a key, and holds two features of the results). q is read from LDS,
+    // which the tiles no longer need (the loop's last barrier is behind every wave). A
+    // row whose scores are numbers has its maximum from above, within 2^kLazy; others
+    // take a pass over the keys for it. Bound: VALU, about 1800 cycles per row and 64
+    // keys. All rows of 32 heads over 8 not finite, 512 of 512 keys: 631 us, 3.2 ms in
+    // the per-row kernel; 300 of 300 of one head: 105 us and 141.
+    float* const qs = reinterpret_cast<float*>(lds + wave * (kAgain * kDh * 4));
     while (again) {
-        const int j = __ffs(again) - 1;
-        again &= again - 1;
-        const int r = w0 + j, lj = min(ke_all, limit_of(r));
-        const int64_t at = ((int64_t)(b * a.Hk * a.G + hk * a.G + r % a.G) * a.Lq + r / a.G) * kDh;
-        auto widen = [&](uint16_t v) { return F16 ? f16_to_f32(v) : bf16_to_f32(v); };
-        auto score = [&](int key) {
-            float s = 0.0f;
-            for (int d = 0; d < kDh; d++)
-                s = fmaf(load_act(a.q, at + d, a.q_dt), widen(a.k[head + (int64_t)key * kDh + d]), s);
-            return s * a.scale;
+        auto widen2 = [](uint32_t u) {
+            if constexpr (F16) {
+                const f16x2_t x = __builtin_bit_cast(f16x2_t, u);
+                return make_float2((float)x.x, (float)x.y);
+            } else {
+                return make_float2(__uint_as_float(u << 16), __uint_as_float(u & 0xFFFF0000u));
+            }
         };
-        float mx = ninf;
-        for (int key = kb + lane; key < lj; key += 64) mx = fmaxf(mx, score(key));
-        mx = wave_max(mx);
-        // a split whose scores are all -inf adds nothing (and without splits the
-        // sum of 0 makes the row NaN)
-        const float sub = mx == ninf ? 0.0f : mx;
-        float ls = 0.0f, x0 = 0.0f, x1 = 0.0f;
-        for (int k0 = kb; k0 < lj; k0 += 64) {
-            const float e = k0 + lane < lj ? (float)exp((double)(score(k0 + lane) - sub)) : 0.0f;
-            ls += e;
-            for (int jj = 0; jj < min(64, lj - k0); jj++) {
-                const float p = __shfl(e, jj, 64);
-                const uint16_t* const vp = a.v + head + (int64_t)(k0 + jj) * kDh;
-                x0 = fmaf(p, widen(vp[lane]), x0);
-                x1 = fmaf(p, widen(vp[lane + 64]), x1);
+        auto row_at = [&](int r) { return ((int64_t)(b * a.Hk * a.G + hk * a.G + r % a.G) * a.Lq + r / a.G) * kDh; };
+        int rr[kAgain], lj[kAgain], count = 0, j = 0;
+        float sub[kAgain];  // the row's maximum, in nats
+        bool pass = false;
+#pragma unroll
+        for (int t = 0; t < kAgain; t++) {
+            if (again) j = __ffs(again) - 1, again &= again - 1, count = t + 1;  // past the last: a repeat
+            rr[t] = w0 + j;
+            lj[t] = min(ke_all, limit_of(rr[t]));
+            sub[t] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(m), j)) * (1.0f / kLog2e);
+            pass |= !finite(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(l), j)));
+            const int64_t at = row_at(rr[t]);
+            qs[t * kDh + lane] = load_act(a.q, at + lane, a.q_dt);
+            qs[t * kDh + lane + 64] = load_act(a.q, at + lane + 64, a.q_dt);
+        }
+        __builtin_amdgcn_wave_barrier();
+        const int end = lj[kAgain - 1];  // the last row's limit is the largest
+        auto scores = [&](int key, float (&s)[kAgain]) {
+            const uint4* const kp = reinterpret_cast<const uint4*>(a.k + head) + (int64_t)min(key, end - 1) * 16;
+            uint4 w[16];
+#pragma unroll
+            for (int i = 0; i < 16; i++) w[i] = kp[i];
+#pragma unroll
+            for (int t = 0; t < kAgain; t++) s[t] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                // one chunk after the other: or all of q is read ahead, and spilled
+                int from = 8 * i;
+                static_assert(kAgain == 8, "the asm's operands");
+                asm volatile("" : "+v"(from), "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]), "+v"(s[4]), "+v"(s[5]),
+                             "+v"(s[6]), "+v"(s[7]));
+                const float2 x0 = widen2(w[i].x), x1 = widen2(w[i].y), x2 = widen2(w[i].z), x3 = widen2(w[i].w);
+#pragma unroll
+                for (int t = 0; t < kAgain; t++) {
+                    const float4 q0 = *reinterpret_cast<const float4*>(qs + t * kDh + from);
+                    const float4 q1 = *reinterpret_cast<const float4*>(qs + t * kDh + from + 4);
+                    s[t] = fmaf(q0.x, x0.x, s[t]), s[t] = fmaf(q0.y, x0.y, s[t]);
+                    s[t] = fmaf(q0.z, x1.x, s[t]), s[t] = fmaf(q0.w, x1.y, s[t]);
+                    s[t] = fmaf(q1.x, x2.x, s[t]), s[t] = fmaf(q1.y, x2.y, s[t]);
+                    s[t] = fmaf(q1.z, x3.x, s[t]), s[t] = fmaf(q1.w, x3.y, s[t]);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < kAgain; t++) s[t] *= a.scale;
+        };
+        float sc[kAgain];
+        if (pass) {
+#pragma unroll
+            for (int t = 0; t < kAgain; t++) sub[t] = ninf;
+            for (int k0 = kb; k0 < end; k0 += 64) {
+                scores(k0 + lane, sc);
+#pragma unroll
+                for (int t = 0; t < kAgain; t++)
+                    if (k0 + lane < lj[t]) sub[t] = fmaxf(sub[t], sc[t]);
+            }
+#pragma unroll
+            for (int t = 0; t < kAgain; t++) sub[t] = wave_max(sub[t]);
+        }
+        float ls[kAgain], r0[kAgain], r1[kAgain], e[kAgain];
+#pragma unroll
+        for (int t = 0; t < kAgain; t++) ls[t] = r0[t] = r1[t] = 0.0f;
+        for (int k0 = kb; k0 < end; k0 += 64) {
+            scores(k0 + lane, sc);
+#pragma unroll
+            for (int t = 0; t < kAgain; t++) {
+                // a split whose scores are all -inf adds nothing (and without splits
+                // the sum of 0 makes the row NaN)
+                const float d = sc[t] - (sub[t] == ninf ? 0.0f : sub[t]);
+                e[t] = k0 + lane < lj[t] ? (float)exp((double)d) : 0.0f;
+                ls[t] += e[t];
+            }
+            const uint32_t* const vp = reinterpret_cast<const uint32_t*>(a.v + head) + lane;
+            for (int j0 = 0; j0 < min(64, end - k0); j0 += 16) {
+                uint32_t vw[16];
+#pragma unroll
+                for (int i = 0; i < 16; i++) vw[i] = vp[(int64_t)min(k0 + j0 + i, end - 1) * 64];
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const float2 x = widen2(vw[i]);
+#pragma unroll
+                    for (int t = 0; t < kAgain; t++) {
+                        if (k0 + j0 + i >= lj[t]) continue;  // not even 0 times the value
+                        const float p =
+                            __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e[t]), j0 + i));
+                        r0[t] = fmaf(p, x.x, r0[t]);
+                        r1[t] = fmaf(p, x.y, r1[t]);
+                    }
+                }
             }
         }
-        ls = wave_sum(ls);
-        if constexpr (SPLIT) {
-            float* const po = a.part_o + ((grow + r) * a.nsplit + blockIdx.y) * kDh;
-            po[lane] = x0;
-            po[lane + 64] = x1;
-            // (m, l) of the row in the units of the others: no 2^7 on p here
-            if (lane == 0) {
-                a.part_ml[((grow + r) * a.nsplit + blockIdx.y) * 2] = mx * kLog2e + kPShift;
-                a.part_ml[((grow + r) * a.nsplit + blockIdx.y) * 2 + 1] = ls;
+#pragma unroll
+        for (int t = 0; t < kAgain; t++) {
+            ls[t] = wave_sum(ls[t]);
+            if (t >= count) break;
+            if constexpr (SPLIT) {
+                const int64_t part = (grow + rr[t]) * a.nsplit + blockIdx.y;
+                *reinterpret_cast<float2*>(a.part_o + part * kDh + 2 * lane) = make_float2(r0[t], r1[t]);
+                // (m, l) in the units of the other rows: no power of two on p here
+                if (lane == 0)
+                    *reinterpret_cast<float2*>(a.part_ml + part * 2) = make_float2(sub[t] * kLog2e + kPShift, ls[t]);
+            } else {
+                const int64_t at = row_at(rr[t]) + 2 * lane;
+                store_y(a.out, at, r0[t] / ls[t], a.out_dt);
+                store_y(a.out, at + 1, r1[t] / ls[t], a.out_dt);
             }
-        } else {
-            store_y(a.out, at + lane, x0 / ls, a.out_dt);
-            store_y(a.out, at + lane + 64, x1 / ls, a.out_dt);
         }
+        __builtin_amdgcn_wave_barrier();
     }
 }
 

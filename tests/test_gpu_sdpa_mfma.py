@@ -167,3 +167,27 @@ def test_sdpa_mfma_scores_of_minus_infinity(hip, oracle, Lk, dead, q_dt, kv_dt):
     assert np.isnan(got[:, 2:]).all()
     ok, dd, sc = rel_ok(got[:, :2], want[:, :2], 1e-5)
     assert ok, (dd, sc)
+
+
+@pytest.mark.parametrize("kv_dt", [F16, BF16])
+@pytest.mark.parametrize("Lk", [70, 700])
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 33, 60])
+def test_sdpa_mfma_rows_again(hip, oracle, n, Lk, kv_dt):
+    """Rows that are not finite are computed again eight at a time: fewer, exactly
+    eight, and more of them, with values that are not finite (one pass over the
+    keys) and a query that is NaN (two)."""
+    Lq = 60
+    q, k, v = _case(1, 1, 1, Lq, Lk, F32, kv_dt)
+    v[0, 0, Lk - n, 5] = -np.inf   # seen by the last n queries, in the tile of others
+    v[0, 0, Lk - n, 64] = np.nan
+    q[0, 0, 11, 3] = np.nan
+    step(f"jh_sdpa rows computed again, n={n} Lk={Lk} kv={kv_dt}")
+    got = hip.Floats(hip.SDPA(_put(hip, q, F32), _put(hip, k, kv_dt), _put(hip, v, kv_dt), D ** -0.5, True))
+    with np.errstate(all="ignore"):
+        want = oracle.sdpa(q, k, v, D ** -0.5, True)
+    seen = [i for i in range(Lq - n, Lq) if i != 11]
+    assert np.isneginf(want[0, 0, seen, 5]).all() and np.isnan(want[0, 0, 11]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    fine = np.isfinite(want)
+    ok, dd, sc = rel_ok(got[fine], want[fine], 1e-5)
+    assert ok, (dd, sc)
