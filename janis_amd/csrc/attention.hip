@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
 #pragma unroll
             for (int n = 0; n < QN; n++) qf[n][kk] = make_uint4(t[0][n], t[1][n], t[2][n], t[3][n]);
         }
-        if (c < 1e-37f) c = 1e-37f;  // a zero scale: equal weights, and masked scores stay -inf
+        if (c < 1e-37f) c = 1e-37f;  // f16, a row of q near zero: equal weights, and masked scores stay -inf
     }
 
     floatx16 o[4];
@@ -547,10 +547,12 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 // Calls the matrix-core kernel takes; others run sdpa_rows_kernel. Its loads
 // and stores are 16 bytes wide (buffers so aligned) with 32-bit offsets inside
-// a head. fp32 keys and values (no model's caches hold them) stay there.
+// a head. fp32 keys and values (no model's caches hold them) stay there, and so
+// does a scale of (next to) zero: times it, the largest scores of bf16 are to
+// vanish, and the factor above is kept from zero.
 bool sdpa_mfma_ok(const void* q, int q_dt, const void* k, const void* v, int kv_dt, const void* out, int64_t B,
-                  int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int64_t Dh) {
-    return Dh == kDh && Lq > 1 && Lk > 0 && (kv_dt == JH_BF16 || kv_dt == JH_F16) &&
+                  int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int64_t Dh, float scale) {
+    return fabsf(scale) >= 1e-30f && Dh == kDh && Lq > 1 && Lk > 0 && (kv_dt == JH_BF16 || kv_dt == JH_F16) &&
            (q_dt == JH_BF16 || q_dt == JH_F32) && Lk < ((int64_t)1 << 22) && Hq / Hk * Lq < ((int64_t)1 << 30) &&
            B * Hk * ((Hq / Hk * Lq + kRows - 1) / kRows) < ((int64_t)1 << 30) && aligned16(q) && aligned16(k) &&
            aligned16(v) && aligned16(out);

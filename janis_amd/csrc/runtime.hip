@@ -744,7 +744,7 @@ int jh_sdpa(jh_ctx* c, const void* q, jh_dtype q_dtype, const void* k, const voi
     const bool fast = jh::sdpa_decode_ok(q_dtype, kv_dtype, Hq, Hk, Lq, Dh);
     if (fast && (!aligned16(k) || !aligned16(v)))
         return fail(c, JH_ERR_INVALID, std::string(op) + ": k and v must be 16-byte aligned");
-    if (jh::sdpa_mfma_ok(q, q_dtype, k, v, kv_dtype, out, B, Hq, Hk, Lq, Lk, Dh)) {
+    if (jh::sdpa_mfma_ok(q, q_dtype, k, v, kv_dtype, out, B, Hq, Hk, Lq, Lk, Dh, scale)) {
         // a split of the keys needs a workspace; where it cannot grow (a stream
         // under capture, no memory) the call runs unsplit
         int64_t nsplit = jh::sdpa_mfma_splits(B, Hq, Hk, Lq, Lk, c->num_cus);

@@ -191,3 +191,15 @@ def test_sdpa_mfma_rows_again(hip, oracle, n, Lk, kv_dt):
     fine = np.isfinite(want)
     ok, dd, sc = rel_ok(got[fine], want[fine], 1e-5)
     assert ok, (dd, sc)
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-38, 1e-30])
+def test_sdpa_mfma_scale_of_nothing(hip, oracle, scale):
+    """Scores of up to 1e38 times a scale of zero, or next to it, are zero (1e-38
+    of them at most 1, 1e-30 far from it: the smallest on the matrix cores)."""
+    q, k, v = _case(1, 2, 1, 20, 90, BF16, BF16)
+    q, k = _round(q * np.float32(1e18), BF16), _round(k * np.float32(1e18), BF16)
+    step(f"jh_sdpa rows scale={scale} of scores of 1e38")
+    got = hip.Floats(hip.SDPA(_put(hip, q, BF16), _put(hip, k, BF16), _put(hip, v, BF16), scale, True, out_dtype=F32))
+    ok, dd, sc = rel_ok(got, oracle.sdpa(q, k, v, scale, True), 1e-5)
+    assert ok, (dd, sc)
