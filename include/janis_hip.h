@@ -274,9 +274,11 @@ JH_API int jh_rope(jh_ctx *ctx, const void *x, jh_dtype x_dtype, int64_t rows, i
  * 90-93) or JH_F32. Lq == 1 with bf16 or f16 k/v, Dh == 128 and Hq/Hk in
  * {1,2,4,8} runs split over the
  * keys (flash-decoding); Lq > 1 with bf16 or f16 k/v and Dh == 128 on the matrix
- * cores at fp32 precision (16-byte aligned buffers; with few rows the keys are
- * split too, through the workspace where it can grow); other shapes a per-row
- * kernel. */
+ * cores at fp32 precision (16-byte aligned buffers). With few rows the keys are
+ * split there too, through the workspace: where it cannot grow (a capture, no
+ * memory) into as many parts as it has room for, so that the speed and the
+ * rounding of a captured call depend on whether the same call ran before the
+ * capture. Other shapes run a per-row kernel. */
 JH_API int jh_sdpa(jh_ctx *ctx, const void *q, jh_dtype q_dtype, const void *k, const void *v,
             jh_dtype kv_dtype, int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk,
             int64_t kv_capacity, int64_t Dh, float scale, int causal, void *out, jh_dtype out_dtype);

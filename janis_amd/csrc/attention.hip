@@ -558,27 +558,28 @@ bool sdpa_mfma_ok(const void* q, int q_dt, const void* k, const void* v, int kv_
            aligned16(v) && aligned16(out);
 }
 
-// Splits of the keys: the count with the least modelled time. On MI355X a 64-key
+size_t sdpa_mfma_workspace_bytes(int64_t B, int64_t Hq, int64_t Lq, int64_t nsplit) {
+    return nsplit > 1 ? sizeof(float) * (size_t)(B * Hq * Lq * nsplit) * (kDh + 2) : 0;
+}
+
+// Splits of the keys: the count with the least modelled time among those whose
+// partials fit max_bytes. On MI355X a 64-key
 // tile of 128 rows took 2.4 us in a block alone on its CU and 3.1 us in each of two
 // that share one, the merge 4 us and its partials (written and read at about 4
 // TB/s). 512 queries of 512 keys stay whole (27 us; in halves 31), 1500 of 4000 too
 // (197; in halves 205), 16 of 4112 take 22 splits (23.5 us; 28.6 with 16 and a merge
 // of one split at a time).
-int64_t sdpa_mfma_splits(int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int num_cus) {
+int64_t sdpa_mfma_splits(int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int num_cus, size_t max_bytes) {
     const int64_t blocks = B * Hk * ((Hq / Hk * Lq + kRows - 1) / kRows), tiles = (Lk + kKeys - 1) / kKeys;
     int64_t best = 1;
     double least = 0;
-    for (int64_t n = 1; n <= tiles && n <= kMaxSplits; n++) {
+    for (int64_t n = 1; n <= tiles && n <= kMaxSplits && sdpa_mfma_workspace_bytes(B, Hq, Lq, n) <= max_bytes; n++) {
         const int64_t per_cu = (blocks * n + num_cus - 1) / num_cus;
         const double work = (3.1 * (double)(per_cu / 2) + 2.4 * (double)(per_cu % 2)) * (double)((tiles + n - 1) / n);
         const double t = work + (n > 1 ? 4.0 + (double)(B * Hq * Lq * n) * (2 * (kDh + 2) * 4) / 4e6 : 0.0);
         if (n == 1 || t < least) best = n, least = t;
     }
     return best;
-}
-
-size_t sdpa_mfma_workspace_bytes(int64_t B, int64_t Hq, int64_t Lq, int64_t nsplit) {
-    return nsplit > 1 ? sizeof(float) * (size_t)(B * Hq * Lq * nsplit) * (kDh + 2) : 0;
 }
 
 Status launch_sdpa_mfma(const void* q, int q_dt, const void* k, const void* v, int kv_dt, void* out, int out_dt,

@@ -356,7 +356,7 @@ Status launch_sdpa(const void* q, int q_dt, const void* k, const void* v, int kv
 // (sdpa_mfma_splits) needs sdpa_mfma_workspace_bytes of workspace.
 bool sdpa_mfma_ok(const void* q, int q_dt, const void* k, const void* v, int kv_dt, const void* out, int64_t B,
                   int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int64_t Dh, float scale);
-int64_t sdpa_mfma_splits(int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int num_cus);
+int64_t sdpa_mfma_splits(int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int num_cus, size_t max_bytes);
 size_t sdpa_mfma_workspace_bytes(int64_t B, int64_t Hq, int64_t Lq, int64_t nsplit);
 Status launch_sdpa_mfma(const void* q, int q_dt, const void* k, const void* v, int kv_dt, void* out, int out_dt,
                         int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int64_t kcap, float scale,

@@ -745,12 +745,14 @@ int jh_sdpa(jh_ctx* c, const void* q, jh_dtype q_dtype, const void* k, const voi
     if (fast && (!aligned16(k) || !aligned16(v)))
         return fail(c, JH_ERR_INVALID, std::string(op) + ": k and v must be 16-byte aligned");
     if (jh::sdpa_mfma_ok(q, q_dtype, k, v, kv_dtype, out, B, Hq, Hk, Lq, Lk, Dh, scale)) {
-        // a split of the keys needs a workspace; where it cannot grow (a stream
-        // under capture, no memory) the call runs unsplit
-        int64_t nsplit = jh::sdpa_mfma_splits(B, Hq, Hk, Lq, Lk, c->num_cus);
-        if (ensure_workspace(c, jh::sdpa_mfma_workspace_bytes(B, Hq, Lq, nsplit), op) != JH_OK) {
+        // a split of the keys needs a workspace; where it cannot grow (a stream under
+        // capture, JH_ERR_INVALID, or no memory) the call takes the best split that
+        // fits the one there is
+        int64_t nsplit = jh::sdpa_mfma_splits(B, Hq, Hk, Lq, Lk, c->num_cus, SIZE_MAX);
+        if (int r = ensure_workspace(c, jh::sdpa_mfma_workspace_bytes(B, Hq, Lq, nsplit), op)) {
+            if (r != JH_ERR_INVALID && r != JH_ERR_OOM) return r;
             c->err.clear();
-            nsplit = 1;
+            nsplit = jh::sdpa_mfma_splits(B, Hq, Hk, Lq, Lk, c->num_cus, c->ws_bytes);
         }
         if (int r = finish(c, jh::launch_sdpa_mfma(q, q_dtype, k, v, kv_dtype, out, out_dtype, B, Hq, Hk, Lq, Lk,
                                                    kv_capacity, scale, causal != 0, nsplit, c->ws, c->stream),

@@ -203,3 +203,29 @@ def test_sdpa_mfma_scale_of_nothing(hip, oracle, scale):
     got = hip.Floats(hip.SDPA(_put(hip, q, BF16), _put(hip, k, BF16), _put(hip, v, BF16), scale, True, out_dtype=F32))
     ok, dd, sc = rel_ok(got, oracle.sdpa(q, k, v, scale, True), 1e-5)
     assert ok, (dd, sc)
+
+
+def test_sdpa_mfma_captured_with_some_workspace(oracle):
+    """Captured on a context whose workspace holds some of the splits' partials,
+    a call takes those: neither the bits of the unsplit sums nor an error."""
+    from janis_amd.engine import HipBackend
+
+    q, k, v = _case(1, 4, 2, 9, 1500, F32, F16)
+    want = oracle.sdpa(q, k, v, D ** -0.5, True)
+    got = []
+    for keys in (None, 150):  # no workspace; one for 150 keys in parts of 64
+        b = HipBackend(0)
+        Q, K, V = _put(b, q, F32), _put(b, k, F16), _put(b, v, F16)
+        if keys:
+            b.SDPA(Q, _put(b, k[:, :, :keys], F16), _put(b, v[:, :, :keys], F16), D ** -0.5, True)
+        arena, out = b.make_arena(1 << 20), []
+        with b.use_arena(arena):
+            step(f"jh_sdpa rows captured after {keys} keys")
+            g = Graph(b, lambda: out.append(b.SDPA(Q, K, V, D ** -0.5, True)))
+        for _ in range(3):
+            g.replay()
+            got.append(b.Floats(out[-1]))
+            ok, dd, sc = rel_ok(got[-1], want, 1e-5)
+            assert ok, (dd, sc)
+        b.Close()
+    assert not np.array_equal(got[0], got[-1])
