@@ -178,31 +178,31 @@ __global__ __launch_bounds__(256) void rms_norm_long_kernel(const void* __restri
         st_act(out, r * d + i, (ld_act(x, r * d + i, x_dt) * inv) * ld_act(w, i, w_dt), out_dt);
 }
 
-// ---- RoPE: one thread per rotated pair and position --------------------------------
+// ---- RoPE: one thread per rotated pair, position and group of heads -----------------
 // The rows at one position (row % L) of a group of `per` heads share a pair's
 // factors: a thread evaluates pow, cos and sin once (in double, as the CPU backend
-// does) and rotates that pair of its group's rows. Bound: the factors and the memory
-// round trips of a thread's rows: 1500 positions of 32 and of 8 heads of 128 take
-// 16.8 us a launch on average on MI355X, 30.8 with the factors evaluated per row.
+// does) and rotates that pair of its group's rows, ROWS of them in flight together
+// (`per` a multiple of ROWS: the loads of a pass in part empty cost calls of one head
+// per thread up to half of their time). Bound: the factors and the memory round trips
+// of a thread's rows. The figures are at the launch.
+template <int ROWS>
 __global__ __launch_bounds__(256) void rope_kernel(const void* __restrict__ x, int x_dt, void* __restrict__ out,
                                                    int out_dt, int64_t rows, int64_t L, int64_t D, int dims,
                                                    int traditional, float base, float scale, int64_t offset,
-                                                   const float* __restrict__ freqs, int64_t per) {
+                                                   const float* __restrict__ freqs, int64_t per, int64_t groups) {
     const int half = dims / 2;
     const int64_t per_row = D - half;  // pairs plus pass-through features
-    const int64_t heads = (rows + L - 1) / L, groups = (heads + per - 1) / per;
-    const int64_t total = groups * L * per_row;
+    const int64_t total = (ROWS == 1 ? rows : groups * L) * per_row;
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
         const int64_t gl = t / per_row;
         const int i = (int)(t - gl * per_row);
         const int64_t g = gl / L, l = gl - g * L;
-        const int64_t h0 = g * per, h1 = min(heads, h0 + per);
+        // this thread's rows: every L-th
+        const int64_t r0 = ROWS == 1 ? gl : g * per * L + l, r1 = ROWS == 1 ? gl + 1 : min(rows, r0 + per * L);
         if (i >= half) {  // features past `dims` pass through
             const int64_t f = dims + (i - half);
-            for (int64_t h = h0; h < h1; h++) {
-                const int64_t o = (h * L + l) * D;
-                if (f < D && h * L + l < rows) st_act(out, o + f, ld_act(x, o + f, x_dt), out_dt);
-            }
+            if (f < D)
+                for (int64_t r = r0; r < r1; r += L) st_act(out, r * D + f, ld_act(x, r * D + f, x_dt), out_dt);
             continue;
         }
         const float inv = freqs ? 1.0f / freqs[i] : (float)pow((double)base, -(double)(2 * i) / (double)dims);
@@ -210,20 +210,26 @@ __global__ __launch_bounds__(256) void rope_kernel(const void* __restrict__ x, i
         const float theta = pos * scale * inv;
         const float c = (float)cos((double)theta), s = (float)sin((double)theta);
         const int64_t j0 = traditional ? 2 * i : i, j1 = traditional ? 2 * i + 1 : i + half;
-        for (int64_t h = h0; h < h1; h += 4) {  // four rows' loads together
-            uint32_t aw[4], bw[4];
+        if constexpr (ROWS == 1) {
+            const float a = ld_act(x, r0 * D + j0, x_dt), b = ld_act(x, r0 * D + j1, x_dt);
+            st_act(out, r0 * D + j0, a * c - b * s, out_dt);
+            st_act(out, r0 * D + j1, a * s + b * c, out_dt);
+            continue;
+        }
+        for (int64_t r = r0; r < r1; r += ROWS * L) {
+            uint32_t aw[ROWS], bw[ROWS];
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int64_t o = min((min(h + q, h1 - 1) * L + l), rows - 1) * D;
+            for (int q = 0; q < ROWS; q++) {
+                const int64_t o = min(r + q * L, rows - 1) * D;
                 aw[q] = ld_word(x, o + j0, x_dt), bw[q] = ld_word(x, o + j1, x_dt);
             }
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int64_t r = (h + q) * L + l;
-                if (h + q >= h1 || r >= rows) break;
-                const float a = word_to_f32(aw[q], x, r * D + j0, x_dt), b = word_to_f32(bw[q], x, r * D + j1, x_dt);
-                st_act(out, r * D + j0, a * c - b * s, out_dt);
-                st_act(out, r * D + j1, a * s + b * c, out_dt);
+            for (int q = 0; q < ROWS; q++) {
+                const int64_t o = (r + q * L) * D;
+                if (r + q * L >= r1) break;
+                const float a = word_to_f32(aw[q], x, o + j0, x_dt), b = word_to_f32(bw[q], x, o + j1, x_dt);
+                st_act(out, o + j0, a * c - b * s, out_dt);
+                st_act(out, o + j1, a * s + b * c, out_dt);
             }
         }
     }
@@ -1573,16 +1579,24 @@ Status launch_rms_norm(const void* x, int x_dt, const void* w, int w_dt, float e
 }
 
 Status launch_rope(const void* x, int x_dt, void* out, int out_dt, int64_t rows, int64_t L, int64_t D, int dims,
-                   bool traditional, float base, float scale, int64_t offset, const float* freqs, hipStream_t st) {
+                   bool traditional, float base, float scale, int64_t offset, const float* freqs, int num_cus,
+                   hipStream_t st) {
     if (rows == 0) return Status::ok();
     L = std::min(L, rows);  // (the position of a row is row % L)
     const int64_t heads = (rows + L - 1) / L, pairs = L * (D - dims / 2);
     if (heads * pairs == 0) return Status::ok();
     // heads per thread: as many as leave four blocks of threads per CU (the factors
-    // are evaluated once per thread; with few positions, one head per thread)
-    const int64_t per = std::max<int64_t>(1, std::min<int64_t>(heads, heads * pairs / (4 * 256 * 256)));
-    hipLaunchKernelGGL(rope_kernel, dim3(grid_for((heads + per - 1) / per * pairs, 256, 16384)), dim3(256), 0, st, x, x_dt,
-                       out, out_dt, rows, L, D, dims, traditional ? 1 : 0, base, scale, offset, freqs, per);
+    // are evaluated once per thread), in whole passes of the kernel. bf16 heads of 128
+    // on MI355X, factors per row / shared: 8 heads at 512 positions 6.0 / 6.0 us (one
+    // head per thread), 32 at 256 9.4 / 7.4 (two), 32 at 512 16.3 / 9.1 (four), 32 at
+    // 1500 39.6 / 15.7.
+    const int64_t most = std::min(heads, heads * pairs / (4 * 256 * (int64_t)num_cus));
+    const int64_t per = most >= 4 ? (most + 1) / 4 * 4 : most >= 2 ? 2 : 1, groups = (heads + per - 1) / per;
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid_for(groups * pairs, 256, 16384)), dim3(256), 0, st, x, x_dt, out, out_dt, rows,
+                           L, D, dims, traditional ? 1 : 0, base, scale, offset, freqs, per, groups);
+    };
+    per >= 4 ? go(rope_kernel<4>) : per == 2 ? go(rope_kernel<2>) : go(rope_kernel<1>);
     return Status::ok();
 }
 

@@ -344,7 +344,8 @@ struct MoeMlpArgs {
 Status launch_rms_norm(const void* x, int x_dt, const void* w, int w_dt, float eps, void* out, int out_dt,
                        int64_t rows, int64_t d, hipStream_t st);
 Status launch_rope(const void* x, int x_dt, void* out, int out_dt, int64_t rows, int64_t L, int64_t D, int dims,
-                   bool traditional, float base, float scale, int64_t offset, const float* freqs, hipStream_t st);
+                   bool traditional, float base, float scale, int64_t offset, const float* freqs, int num_cus,
+                   hipStream_t st);
 bool sdpa_decode_ok(int q_dt, int kv_dt, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Dh);
 int64_t sdpa_splits(int64_t B, int64_t Hk, int64_t Lk, int num_cus);
 size_t sdpa_workspace_bytes(int q_dt, int kv_dt, int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk,

@@ -722,7 +722,7 @@ int jh_rope(jh_ctx* c, const void* x, jh_dtype x_dtype, int64_t rows, int64_t L,
     if (rows == 0) return JH_OK;
     if (!x || !out) return fail(c, JH_ERR_INVALID, std::string(op) + ": null pointer");
     if (int r = finish(c, jh::launch_rope(x, x_dtype, out, out_dtype, rows, L, D, dims, traditional != 0, base, scale,
-                                     offset, freqs, c->stream),
+                                     offset, freqs, c->num_cus, c->stream),
                   op)) return r;
     return check_values(c, op, out, out_dtype, rows * D);
 }

@@ -110,10 +110,13 @@ def test_copy_broadcast_and_reverse(hip):
 
 @pytest.mark.parametrize("heads,L,D,dims,traditional", [(1, 1, 128, 128, False), (40, 700, 128, 128, False),
                                                         (33, 300, 96, 64, False), (6, 301, 64, 64, True),
-                                                        (130, 70, 128, 32, False)])
+                                                        (130, 70, 128, 32, False),
+                                                        (39, 700, 128, 128, False), (67, 500, 128, 128, True),
+                                                        (8, 512, 128, 128, False)])
 @pytest.mark.parametrize("dt", [F32, BF16])
 def test_rope_head_groups(hip, oracle, heads, L, D, dims, traditional, dt):
-    """Heads that share a position's factors, in whole groups and not."""
+    """Heads that share a position's factors (one, two, four and eight per thread),
+    in whole groups and not."""
     rng = np.random.default_rng(heads + L)
     raw, x = _bits(rng.standard_normal((1, heads, L, D)), dt)
     t = hip.FromRaw(dt, raw, *raw.shape)
