@@ -862,16 +862,26 @@ void run_tile(const MoeArgs& a, bool sb_f16, int mode, int64_t max_u, hipStream_
 // kMfmaPairsPerExpert pairs per expert of the stack, groups of 64 or 128, every K
 // of the tiles (a multiple of 256), x within a buffer resource's 2 GiB, scales and
 // biases 8-byte aligned (a lane reads a step's four at once, the dot products read
-// them one by one; every expert's and row's start is then aligned too). Measured
-// on MI355X, jh_moe_route + jh_moe_swiglu of 128 experts (2048 x 768, top 8), dot
-// products against matrix cores: 16 tokens 88 / 105 us, 24 109 / 114, 32 126 /
-// 119, 48 159 / 128, 500 1004 / 187, 2000 3831 / 465. The line is at 32 tokens,
-// 2 pairs per expert.
+// them one by one; every expert's and row's start is then aligned too) -- and enough
+// products to pay for the K steps that a block of that kernel takes one after the
+// other, about 1.1 us each with one stack and 2 with two, however few pairs it has.
+// The line for that is in rows of output (pairs times rows of the stacks). Measured
+// on MI355X, us a launch on the dot products / the matrix cores, at 8 to 64 experts:
+//   one stack   512 x 1024  48 pairs  8.0 / 8.7    64 pairs  9.1 / 8.9   128 pairs 13.1 / 9.0
+//   (28 K rows) 768 x 2048  48 pairs 10.8 / 13.0   64 pairs 12.5 / 13.2   96 pairs 15.4 / 13.4
+//   (60000)     256 x 4096 192 pairs 19.1 / 20.8  256 pairs 23.2 / 21.2
+//   two stacks  512 x 1024  64 pairs 10.5 / 12.8   80 pairs 12.2 / 12.9  128 pairs 15.6 / 13.2
+//   (80000      768 x 2048  48 pairs 15.8 / 20.6   64 pairs 19.3 / 20.7   96 pairs 23.2 / 20.6
+//    + 10 K)   1536 x 4096  40 pairs 40.7 / 35.2
+// and at 2 pairs per expert of 128, above the line: 768 x 2048 twice 58.2 / 53.0, the
+// down product 2048 x 768 41.0 / 35.3; 512 x 1024 twice 23.1 / 20.7, down 15.9 / 14.9.
 constexpr int64_t kMfmaPairsPerExpert = 2;
-bool moe_mfma_ok(const MoeArgs& a, int64_t P, int mode) {
+bool moe_mfma_ok(const MoeArgs& a, int64_t P, int mode, int stacks) {
     const uintptr_t sb = reinterpret_cast<uintptr_t>(a.s[0]) | reinterpret_cast<uintptr_t>(a.s[1]) |
                          reinterpret_cast<uintptr_t>(a.b[0]) | reinterpret_cast<uintptr_t>(a.b[1]);
-    return (sb & 7u) == 0 && mode == MODE_WS && (a.gs_log2 == 6 || a.gs_log2 == 7) && P % 32 == 0 &&
+    const int64_t K = 8 * P, rows = (int64_t)a.n_pairs * a.N * stacks;
+    const int64_t line = stacks == 1 ? std::min<int64_t>(28 * K, 60000) : 80000 + 10 * K;
+    return (sb & 7u) == 0 && mode == MODE_WS && (a.gs_log2 == 6 || a.gs_log2 == 7) && P % 32 == 0 && rows >= line &&
            a.n_pairs >= kMfmaPairsPerExpert * a.E && (int64_t)a.n_pairs * P * 16 < ((int64_t)1 << 31);
 }
 
@@ -885,7 +895,7 @@ void run_mfma(const MoeArgs& a, int64_t P, bool sb_f16, int64_t max_u, hipStream
 
 template <int EPI>
 bool run_fast(const MoeArgs& a, int64_t P, bool sb_f16, int mode, int64_t max_u, hipStream_t st) {
-    if (moe_mfma_ok(a, P, mode)) {
+    if (moe_mfma_ok(a, P, mode, EPI == EPI_SWIGLU ? 2 : 1)) {
         run_mfma<EPI>(a, P, sb_f16, max_u, st);
         return true;
     }

@@ -34,11 +34,14 @@ def _buckets(sizes, k_slots, seed):
 
 # buckets around the tile's 32 and 64 pairs, an unused expert, several tiles of
 # one bucket; rows that are no multiple of a wave's 32 or a block's 128; the
-# shortest K and one that is not a power of two; both groups, both scale types
+# shortest K and one that is not a power of two; both groups, both scale types.
+# (Calls of fewer than 28 K rows of output stay on the dot products: three here,
+# and each of them with more rows.)
 @pytest.mark.parametrize("sizes,slots,n,k,gs,sb", [
     ((1, 31, 32, 0), 4, 128, 256, 64, BF16), ((33, 63, 64, 4), 4, 33, 768, 64, F16),
     ((65, 0, 130, 1, 4), 8, 100, 512, 128, BF16), ((2, 2, 2, 2, 128), 8, 257, 2048, 64, BF16),
-    ((40, 40), 1, 160, 1536, 128, F16)])
+    ((40, 40), 1, 160, 1536, 128, F16), ((33, 63, 64, 4), 4, 161, 768, 64, F16),
+    ((2, 2, 2, 2, 128), 8, 433, 2048, 64, BF16), ((40, 40), 1, 545, 1536, 128, F16)])
 def test_gather_mfma(hip, oracle, sizes, slots, n, k, gs, sb):
     E, idx = len(sizes), _buckets(sizes, slots, n + k)
     q = synth.quant_linear(810 + n, n, k, gs, lead=(E,))
@@ -72,10 +75,11 @@ def test_moe_swiglu_mfma(hip, oracle, sizes, H, I, gs, out_dtype):
     assert np.array_equal(first.view(np.uint32), again.view(np.uint32))
 
 
-def test_gather_mfma_rows_apart(hip, oracle):
+@pytest.mark.parametrize("n", [64, 232])
+def test_gather_mfma_rows_apart(hip, oracle, n):
     """A pair whose x holds a NaN or an infinity, and one with an index outside
     the stack, leave the other pairs of their bucket and tile alone."""
-    E, n, k = 2, 64, 512
+    E, k = 2, 512
     idx = _buckets((40, 24), 4, 3)
     q = synth.quant_linear(840, n, k, lead=(E,))
     w, s, b = upload_quant(hip, q)
@@ -124,11 +128,12 @@ def test_moe_route_sizes(hip, oracle, E, k):
     assert np.array_equal(got_i[6:], np.tile(np.arange(k, dtype=np.int32), (2, 1))) and np.isnan(got_s[6:]).all()
 
 
+@pytest.mark.parametrize("n", [64, 232])
 @pytest.mark.parametrize("gs", [64, 128])
-def test_gather_scales_at_two_bytes(hip, oracle, gs):
+def test_gather_scales_at_two_bytes(hip, oracle, gs, n):
     """Scales and biases that start at an odd element (2-byte aligned) keep
     their results: such calls stay on the dot products."""
-    E, n, k = 2, 64, 512
+    E, k = 2, 512
     idx = _buckets((40, 24), 4, 5)
     q = synth.quant_linear(850, n, k, gs, lead=(E,))
     w = upload_quant(hip, q)[0]
@@ -143,3 +148,41 @@ def test_gather_scales_at_two_bytes(hip, oracle, gs):
                                          out_dtype=F32))
     ok, d, sc = rel_ok(y, oracle.gather_quant_matmul(x, q.w, q.s, q.b, idx, gs), 1e-5)
     assert ok, (d, sc)
+
+
+# either side of the lines between the dot products and the matrix cores: 28 K rows
+# of output for one stack, 80000 + 10 K for two (pairs times rows)
+@pytest.mark.parametrize("n,k", [(335, 768), (336, 768), (223, 512), (224, 512), (895, 2048), (896, 2048)])
+def test_gather_at_the_line(hip, oracle, n, k):
+    E, idx = 8, _buckets((9, 3, 0, 17, 1, 16, 8, 10), 4, 7)
+    q = synth.quant_linear(860 + n, n, k, lead=(E,))
+    xb, x = synth.activations(861, (16, 1, 1, k))
+    step(f"jh_gather_quant_matmul 64 pairs n={n} k={k}")
+    y = hip.Floats(hip.GatherQuantMatmul(hip.FromBF16Bits(xb, 16, 1, 1, k), *upload_quant(hip, q), hip.FromInt32(idx), True,
+                                         64, 4, out_dtype=F32))
+    ok, d, sc = rel_ok(y, oracle.gather_quant_matmul(x, q.w, q.s, q.b, idx, 64), 1e-5)
+    assert ok, (d, sc)
+
+
+@pytest.mark.parametrize("I", [512, 768])
+@pytest.mark.parametrize("slots", [4, 9, 16, 17])
+def test_moe_swiglu_slots(hip, oracle, I, slots):
+    """More than eight slots per token (the sum over slots takes eight at a time),
+    an index outside the stack among them; gate and up on the dot products or on
+    the matrix cores, down on the matrix cores."""
+    E, H, T = 18, 512, 6
+    rng = np.random.default_rng(slots)
+    idx = np.stack([rng.permutation(E)[:slots] for _ in range(T)]).astype(np.int32)
+    qs = [synth.quant_linear(870 + i, *(I, H) if i < 2 else (H, I), 64, lead=(E,)) for i in range(3)]
+    sc = rng.random(idx.shape).astype(np.float32)
+    xb, x = synth.activations(871, (T, H))
+    want = oracle.moe_apply(x, *[(q.w, q.s, q.b) for q in qs], idx, sc, 64)
+    idx[2, slots - 1] = E
+    st = [upload_quant(hip, q) for q in qs]
+    step(f"jh_moe_swiglu slots={slots} I={I}")
+    got = hip.Floats(hip.MoeSwiGLU(hip.FromBF16Bits(xb, T, H), *st, hip.FromInt32(idx), hip.FromFloats(sc), 64, 4,
+                                   out_dtype=F32))
+    keep = np.arange(T) != 2
+    assert np.isnan(got.reshape(T, H)[2]).all()
+    ok, d, s = rel_ok(got.reshape(T, H)[keep], want.reshape(T, H)[keep], 1e-2)
+    assert ok, (d, s)
