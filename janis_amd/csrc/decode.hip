@@ -97,38 +97,61 @@ __device__ float block_sum256(float v, float* red) {
 // no branch on their types (no load waits on an earlier one, nor the weights on the
 // reduction), squared and summed, then scaled from the registers: x is read once.
 // Rows of up to 1024 take one wave each (per-head norms), longer rows one block of
-// 256 threads. One fp32 row of 4096 takes 5.1 us on MI355X, 9.2 with the weights
-// loaded after the sum.
+// 256 threads, each length the instance with the fewest registers that hold it: the
+// ones past the row's end are loaded all the same (its last element again). On MI355X,
+// weights loaded after the sum / 64-bit addresses per load and fewer instances / now:
+// one fp32 row of 4096 6.7 / 5.1 / 4.8 us, bf16 48000 x 128 12.7 / 13.2 / 12.5, 20000 x
+// 300 14.0 / 18.6 / 10.9, 2048 x 12288 125 / 121 / 42.
+// A run of elements read as aligned 32-bit words (ld_word's way) at 32-bit offsets
+// from one base, which is the same for every lane of a wave.
+struct Words {
+    const char* base;
+    uint32_t skip, shift;  // bytes from base to element 0; log2 of an element's bytes
+    __device__ __forceinline__ Words(const void* p, int64_t first, int dt) {
+        shift = dt == JH_F32 ? 2 : 1;
+        const char* const e = static_cast<const char*>(p) + (first << shift);
+        skip = (uint32_t)(reinterpret_cast<uintptr_t>(e) & 3);
+        base = e - skip;
+    }
+    __device__ __forceinline__ uint32_t load(uint32_t i) const {
+        return *reinterpret_cast<const uint32_t*>(base + (((i << shift) + skip) & ~3u));
+    }
+    __device__ __forceinline__ float value(uint32_t word, uint32_t i, int dt) const {
+        if (dt == JH_F32) return __uint_as_float(word);
+        const uint16_t h = (uint16_t)(((i << shift) + skip) & 2 ? word >> 16 : word);
+        return dt == JH_BF16 ? bf16_to_f32(h) : f16_to_f32(h);
+    }
+};
+
 template <int PER>  // elements per lane (wave kernel) or per thread (block kernel)
 struct NormRow {
     uint32_t xw[PER], ww[PER];
     float v[PER];
-    __device__ __forceinline__ void load(const void* x, int x_dt, int64_t base, const void* w, int w_dt, int64_t d,
-                                         int t, int stride) {
+    __device__ __forceinline__ void load(const Words& x, const Words& w, uint32_t d, uint32_t t, uint32_t stride) {
 #pragma unroll
         for (int e = 0; e < PER; e++) {
-            const int64_t i = min(t + (int64_t)e * stride, d - 1);
-            xw[e] = ld_word(x, base + i, x_dt);
-            ww[e] = ld_word(w, i, w_dt);
+            const uint32_t i = min(t + e * stride, d - 1);
+            xw[e] = x.load(i);
+            ww[e] = w.load(i);
         }
     }
     // this lane's sum of squares
-    __device__ __forceinline__ float squares(const void* x, int x_dt, int64_t base, int64_t d, int t, int stride) {
+    __device__ __forceinline__ float squares(const Words& x, int x_dt, uint32_t d, uint32_t t, uint32_t stride) {
         float ss = 0.0f;
 #pragma unroll
         for (int e = 0; e < PER; e++) {
-            const int64_t i = t + (int64_t)e * stride;
-            v[e] = i < d ? word_to_f32(xw[e], x, base + i, x_dt) : 0.0f;
+            const uint32_t i = t + e * stride;
+            v[e] = i < d ? x.value(xw[e], i, x_dt) : 0.0f;
             ss = fmaf(v[e], v[e], ss);
         }
         return ss;
     }
-    __device__ __forceinline__ void store(void* out, int out_dt, int64_t base, const void* w, int w_dt, int64_t d, int t,
-                                          int stride, float inv) {
+    __device__ __forceinline__ void store(void* out, int out_dt, int64_t base, const Words& w, int w_dt, uint32_t d,
+                                          uint32_t t, uint32_t stride, float inv) {
 #pragma unroll
         for (int e = 0; e < PER; e++) {
-            const int64_t i = t + (int64_t)e * stride;
-            if (i < d) st_act(out, base + i, (v[e] * inv) * word_to_f32(ww[e], w, i, w_dt), out_dt);
+            const uint32_t i = t + e * stride;
+            if (i < d) st_act(out, base + i, (v[e] * inv) * w.value(ww[e], i, w_dt), out_dt);
         }
     }
 };
@@ -138,14 +161,15 @@ __global__ __launch_bounds__(256) void rms_norm_wave_kernel(const void* __restri
                                                             const void* __restrict__ w, int w_dt, float eps,
                                                             void* __restrict__ out, int out_dt, int64_t rows,
                                                             int64_t d) {
-    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t r = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (r >= rows) return;
+    const Words xs(x, r * d, x_dt), ws(w, 0, w_dt);
     NormRow<PER> n;
-    n.load(x, x_dt, r * d, w, w_dt, d, lane, 64);
-    const float ss = wave_sum(n.squares(x, x_dt, r * d, d, lane, 64));
+    n.load(xs, ws, (uint32_t)d, lane, 64);
+    const float ss = wave_sum(n.squares(xs, x_dt, (uint32_t)d, lane, 64));
     const float inv = 1.0f / (float)sqrt((double)(ss / (float)d + eps));
-    n.store(out, out_dt, r * d, w, w_dt, d, lane, 64, inv);
+    n.store(out, out_dt, r * d, ws, w_dt, (uint32_t)d, lane, 64, inv);
 }
 
 template <int PER>
@@ -154,11 +178,12 @@ __global__ __launch_bounds__(256) void rms_norm_block_kernel(const void* __restr
                                                              void* __restrict__ out, int out_dt, int64_t d) {
     __shared__ float red[4];
     const int64_t r = blockIdx.x;
+    const Words xs(x, r * d, x_dt), ws(w, 0, w_dt);
     NormRow<PER> n;
-    n.load(x, x_dt, r * d, w, w_dt, d, threadIdx.x, 256);
-    const float ss = block_sum256(n.squares(x, x_dt, r * d, d, threadIdx.x, 256), red);
+    n.load(xs, ws, (uint32_t)d, threadIdx.x, 256);
+    const float ss = block_sum256(n.squares(xs, x_dt, (uint32_t)d, threadIdx.x, 256), red);
     const float inv = 1.0f / (float)sqrt((double)(ss / (float)d + eps));
-    n.store(out, out_dt, r * d, w, w_dt, d, threadIdx.x, 256, inv);
+    n.store(out, out_dt, r * d, ws, w_dt, (uint32_t)d, threadIdx.x, 256, inv);
 }
 
 // Rows longer than 256 * 64 elements: two passes over x.
@@ -1570,9 +1595,13 @@ Status launch_rms_norm(const void* x, int x_dt, const void* w, int w_dt, float e
     auto block = [&](auto k) { hipLaunchKernelGGL(k, bg, dim3(256), 0, st, x, x_dt, w, w_dt, eps, out, out_dt, d); };
     if (d <= 128) wave(rms_norm_wave_kernel<2>);
     else if (d <= 256) wave(rms_norm_wave_kernel<4>);
+    else if (d <= 512) wave(rms_norm_wave_kernel<8>);
     else if (d <= 1024) wave(rms_norm_wave_kernel<16>);
+    else if (d <= 2048) block(rms_norm_block_kernel<8>);
     else if (d <= 4096) block(rms_norm_block_kernel<16>);
+    else if (d <= 6144) block(rms_norm_block_kernel<24>);
     else if (d <= 8192) block(rms_norm_block_kernel<32>);
+    else if (d <= 12288) block(rms_norm_block_kernel<48>);
     else if (d <= 16384) block(rms_norm_block_kernel<64>);
     else block(rms_norm_long_kernel);
     return Status::ok();

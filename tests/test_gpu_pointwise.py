@@ -133,16 +133,23 @@ def test_rope_head_groups(hip, oracle, heads, L, D, dims, traditional, dt):
             np.testing.assert_array_equal(hip.Floats(out), got.reshape(-1, D)[:rows])
 
 
-@pytest.mark.parametrize("rows,d", [(3, 1), (5, 63), (2, 129), (9, 1024), (2, 1025), (3, 4095), (1, 12288), (2, 16385)])
+@pytest.mark.parametrize("rows,d", [(3, 1), (5, 63), (2, 128), (2, 129), (3, 256), (3, 257), (5, 300), (2, 512), (2, 513),
+                                    (9, 1024), (2, 1025), (2, 2048), (2, 2049), (3, 4095), (2, 4097), (2, 6144), (2, 6145),
+                                    (2, 8192), (2, 8193), (1, 12288), (1, 12289), (1, 16384), (2, 16385)])
 @pytest.mark.parametrize("x_dt,w_dt", [(F32, BF16), (BF16, F16), (BF16, F32)])
-def test_rms_norm_lengths(hip, oracle, rows, d, x_dt, w_dt):
-    """Row lengths at the ends of each kernel's range, odd ones among them."""
+def test_rms_norm_lengths(hip, rows, d, x_dt, w_dt):
+    """Row lengths at the ends of each kernel's range, odd ones among them. The first
+    and the last element of a row hold most of its sum of squares, so that one left
+    out or taken twice shows at every length."""
     rng = np.random.default_rng(rows * d)
-    rx, x = _bits(rng.standard_normal((rows, d)), x_dt)
+    x = rng.standard_normal((rows, d))
+    x[:, 0], x[:, -1] = np.sqrt(d), -1.5 * np.sqrt(d)
+    rx, x = _bits(x, x_dt)
     rw, w = _bits(1 + 0.1 * rng.standard_normal(d), w_dt)
     step(f"jh_rms_norm rows={rows} d={d} x={x_dt} w={w_dt}")
     got = hip.Floats(hip.RMSNorm(hip.FromRaw(x_dt, rx, rows, d), hip.FromRaw(w_dt, rw, d), 1e-6, out_dtype=F32))
-    want = oracle.rms_norm(x, w, 1e-6)
-    # the oracle adds the d squares one after another, each sum rounded: up to
-    # d * 2^-24 of it, half that in its root (the kernel adds at most 65 in a row)
-    assert np.abs(got - want).max() <= (2.0 ** -22 + 0.5 * d * 2.0 ** -24) * np.abs(want).max()
+    x64 = x.astype(np.float64)
+    want = x64 / np.sqrt((x64 ** 2).mean(-1, keepdims=True) + 1e-6) * w
+    # a thread adds up to 65 squares one after another and 8 sums follow: 73 * 2^-24
+    # of the sum, half that in its root; then a quotient, a root and two products
+    assert (np.abs(got - want) <= (37 + 5) * 2.0 ** -24 * np.abs(want)).all()
