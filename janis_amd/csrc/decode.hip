@@ -1268,9 +1268,10 @@ __global__ __launch_bounds__(64) void xcc_probe_kernel(int* out) {
 
 // ---- elementwise -----------------------------------------------------------------
 // fl32(exp(x)) evaluated in fp64 as the CPU backend does: x = n ln 2 + r, the
-// Taylor polynomial of e^r to r^11 (|r| <= 0.347: 2^-46 of the result, so the
-// rounding to fp32 is what is left), scaled by 2^n. 19 fp64 instructions where
-// the library's exp, good to fp64, takes about twice as many. The argument is
+// Taylor polynomial of e^r to r^11 (|r| <= 0.347: 2^-46 of the result), scaled by
+// 2^n. 19 fp64 instructions where the library's exp, good to fp64, takes about twice
+// as many. Of all fp32 arguments two (-1.0149802 and -14.56709) get the fp32 value next
+// to that of the exact exponential, and SiLU of neither changes. The argument is
 // clamped to where fl32(exp) is already 0 or infinite; NaN stays NaN.
 __device__ __forceinline__ float exp_fp64(float x) {
     const double t = (double)fminf(fmaxf(x, -110.0f), 90.0f);
@@ -1345,8 +1346,22 @@ __global__ __launch_bounds__(256) void elementwise_kernel(int op, const void* __
         }
         tail = n / 8 * 8;
     }
-    for (int64_t i = tail + first; i < n; i += stride)
-        st_act(out, i, elementwise_one(op, ld_act(a, i, a_dt), op == JH_OP_SILU ? 0.0f : ld_act(b, i, b_dt)), out_dt);
+    const bool f32 = a_dt == JH_F32 && b_dt == JH_F32 && op != JH_OP_SILU;
+    for (int64_t i = tail + first; i < n; i += stride) {
+        float x, y, r;
+        if (f32) {
+            x = static_cast<const float*>(a)[i], y = static_cast<const float*>(b)[i];  // requested together
+        } else {
+            x = ld_act(a, i, a_dt);
+        }
+        if (op == JH_OP_SILU) {
+            r = x / (1.0f + exp_fp64(-x));
+        } else {
+            if (!f32) y = ld_act(b, i, b_dt);
+            r = op == JH_OP_ADD ? x + y : op == JH_OP_MUL ? x * y : (x / (1.0f + exp_fp64(-x))) * y;
+        }
+        st_act(out, i, r, out_dt);
+    }
 }
 
 // ---- Argmax: first index of the maximum; blocks take chunks, one block merges ----
@@ -1911,11 +1926,13 @@ Status launch_rope_table(int dims, float base, float scale, int64_t pos, const f
 
 // In pieces of 8 from this many elements, below one by one: with fewer the chip is
 // not full and a thread's eight elements (for SiLU its eight exponentials) come one
-// after the other. bf16 on MI355X, one by one / in pieces: Add of 12288 elements
-// 2.4 / 3.0 us, 400000 3.1 / 3.1, 800000 3.9 / 3.4, 2^22 11.8 / 6.1; SiLU(a) * b of
-// 98304 3.1 / 4.6, 786432 5.5 / 5.1, 1228800 6.2 / 6.0, 2^22 13.2 / 9.8 (SiLU one by
-// one measured with the library's exponential).
-constexpr int64_t kAddVecMin = (int64_t)1 << 19, kSiluVecMin = (int64_t)1 << 20;
+// after the other. us on MI355X, one by one / in pieces, bf16 and fp32: Add of 12288
+// elements 2.4 / 2.9 and 2.3 / 2.6, 400000 3.1 / 3.0 and 2.9 / 2.9, 524288 3.3 / 3.1 and
+// 3.1 / 3.0, 2^22 12.1 / 6.0 and 11.7 / 9.1; SiLU(a) 800000 3.9 / 4.5 and 4.0 / 4.3,
+// 1228800 4.9 / 5.1 and 5.1 / 5.0, 1500000 5.6 / 5.2 and 5.8 / 5.3, 2^22 12.1 / 9.6 and
+// 11.9 / 9.9; SiLU(a) * b 800000 4.3 / 4.7 and 4.1 / 4.5, 1228800 5.5 / 5.2 and 5.2 / 5.2,
+// 2^22 13.3 / 9.9 and 13.1 / 12.0.
+constexpr int64_t kAddVecMin = (int64_t)1 << 19, kSiluVecMin = (int64_t)5 << 18;
 
 Status launch_elementwise(int op, const void* a, int a_dt, const void* b, int b_dt, void* out, int out_dt, int64_t n,
                           hipStream_t st) {

@@ -33,8 +33,9 @@ def _at(hip, raw, dt, shift):
     return t, t.ptr + shift * SIZE[dt]
 
 
-# (Add and Mul move pieces of 8 from 2^19 elements on, SiLU from 2^20)
-@pytest.mark.parametrize("n", [1, 7, 8, 2049, 12288, (1 << 19) + 5, (1 << 20) - 1, (1 << 20) + 3])
+# (Add and Mul move pieces of 8 from 2^19 elements on, SiLU from 5 * 2^18)
+@pytest.mark.parametrize("n", [1, 7, 8, 2049, 12288, (1 << 19) + 5, (1 << 20) - 1, (1 << 20) + 3, (5 << 18) - 1,
+                               (5 << 18) + 3])
 @pytest.mark.parametrize("a_dt,b_dt,o_dt,shift", [(F32, F32, F32, 0), (BF16, BF16, BF16, 0), (F32, BF16, BF16, 0),
                                                   (BF16, F32, F32, 0), (F32, F32, F32, 1), (BF16, BF16, F32, 3)])
 def test_elementwise_sizes(hip, oracle, n, a_dt, b_dt, o_dt, shift):
