@@ -499,7 +499,7 @@ class HipBackend:
     def Reshape(self, x: Tensor, *shape) -> Tensor:
         """engine.Backend.Reshape: a view of the same memory when x is dense (one
         -1 allowed), else of a dense copy."""
-        shape = list(shape)
+        shape = [int(d) for d in shape]  # (a product of numpy's 32-bit integers would wrap)
         if shape.count(-1) == 1:
             known = math.prod([d for d in shape if d != -1])
             shape[shape.index(-1)] = x.numel // known if known else 0

@@ -86,3 +86,16 @@ def test_product_does_not_import_the_oracle():
                         assert (node.module or "").split(".")[0] != "oracle", f
             if f.endswith((".hip", ".hpp", ".cpp", ".h")):
                 assert "janis_oracle" not in open(os.path.join(dirpath, f)).read(), f
+
+
+def test_reshape_counts_elements_in_python_integers():
+    """Dimensions of numpy's 32-bit integers, whose product wraps at 2^31, reshape a
+    tensor of more elements than that. (A view: no memory is touched.)"""
+    np = pytest.importorskip("numpy")
+    from janis_amd import engine
+
+    b = object.__new__(engine.HipBackend)
+    x = engine.Tensor(None, 256, (151936, 16384), engine.BF16, owned=False)
+    for shape in ((151936 * 4, 4096), (-1, 4096), (16384, 151936)):
+        y = b.Reshape(x, *(np.int32(d) for d in shape))
+        assert y.numel == x.numel and y.ptr == x.ptr and all(type(d) is int for d in y.shape)
