@@ -56,8 +56,13 @@ constexpr int kKeys = 64;   // keys per tile
 constexpr int kTileBytes = kKeys * kDh * 2;
 constexpr int kAgain = 8;    // rows computed again together
 constexpr float kLog2e = 1.44269504088896340736f;
-constexpr float kPShift = 13.0f;  // p is held as p * 2^13
-constexpr float kLazy = 2.0f;     // a row's maximum is moved when it grew by more than this (log2)
+// p is held as p * 2^kPShift, and a row's maximum is moved when it grew by more than
+// kLazy (log2): f16 terms have nothing below 2^-24 and nothing past 2^16, so p is kept
+// high there; bf16 terms have fp32's range, and each move costs 64 products.
+template <bool F16>
+constexpr float kPShift = F16 ? 13.0f : 7.0f;
+template <bool F16>
+constexpr float kLazy = F16 ? 2.0f : 8.0f;
 
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
@@ -263,7 +268,7 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
 #pragma unroll
         for (int r = 0; r < 16; r++) mt = fmaxf(mt, fmaxf(s[0][r], s[1][r]));
         mt = pair32<true>(mt) * c;
-        if (__any(mt > m + kLazy)) {
+        if (__any(mt > m + kLazy<F16>)) {
             const float mn = fmaxf(m, mt);
             const float f = mn == ninf ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
             l *= f;
@@ -273,7 +278,7 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
                 for (int r = 0; r < 16; r++) o[t][r] *= f;
             m = mn;
         }
-        const float neg = m == ninf ? 0.0f : kPShift - m;
+        const float neg = m == ninf ? 0.0f : kPShift<F16> - m;
         float ls = 0.0f;
 #pragma unroll
         for (int g = 0; g < 2; g++)
@@ -493,7 +498,7 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
                 *reinterpret_cast<float2*>(a.part_o + part * kDh + 2 * lane) = make_float2(r0[t], r1[t]);
                 // (m, l) in the units of the other rows: no power of two on p here
                 if (lane == 0)
-                    *reinterpret_cast<float2*>(a.part_ml + part * 2) = make_float2(sub[t] * kLog2e + kPShift, ls[t]);
+                    *reinterpret_cast<float2*>(a.part_ml + part * 2) = make_float2(sub[t] * kLog2e + kPShift<F16>, ls[t]);
             } else {
                 const int64_t at = row_at(rr[t]) + 2 * lane;
                 store_y(a.out, at, r0[t] / ls[t], a.out_dt);
