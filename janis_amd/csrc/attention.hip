@@ -38,13 +38,19 @@
 // whose result is not finite is computed again with that kernel's arithmetic over
 // the block's keys, and that result stands.
 //
-// Bound: the matrix cores, with the softmax's VALU work beside them: per 32
-// rows x 64 keys, 16 MFMAs for each q term and 16 for each p term (512 cycles
-// each 16) against ~1100 cycles of VALU. K/V tiles come through registers into
+// Per 32 rows x 64 keys a wave issues 16 MFMAs for each q term and 16 for each p term
+// (512 cycles each 16) and ~1100 cycles of VALU. K/V tiles come through registers into
 // two LDS buffers (64 KiB: two blocks per CU), the next tile's loads in flight
-// during the current one. Measured on MI355X, 32 heads over 8 (calls from the
-// host, the per-row kernel before): 512 queries of 512 keys 3433 -> 46 us (fp32
-// q, f16 keys), 1500 of 4000 144.9 ms -> 222 us (bf16), 16 of 4112 2.9 ms -> 37 us.
+// during the current one. What bounds it, by counters (32 heads over 8, 1500 queries
+// of 4000 bf16 keys): the MFMA pipes are busy 33 % of the time and VALU 31, one after
+// the other at one or two waves per SIMD (376 blocks on 256 CUs); the waves issue in
+// 41 % of their cycles, are ready behind another instruction in 36 and wait for
+// memory, LDS or barriers in 23. LDS is active 31 % of the time, half of that in bank
+// conflicts. 512 queries of 512 keys are 128 blocks: half of the CUs idle, the MFMA
+// pipes 5 % busy.
+// Measured on MI355X (replayed graphs; the per-row kernel before): 512 queries of
+// 512 keys 3230 -> 30 us (fp32 q, f16 keys), 1500 of 4000 143 ms -> 220 us (bf16), 16 of
+// 4112 2.8 ms -> 26 us (fp32 q, f16 keys).
 #include "jh_common.hpp"
 
 namespace jh {
@@ -128,7 +134,7 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
     constexpr int PN = F16 ? 2 : 3;
     // two slots of a key tile [64][128] (16-byte chunk c of key k at c ^ (k % 16))
     // and a value tile transposed, [128][64] (4-key chunk s of feature d at
-    // s ^ (d / 2 % 16)): every fragment read below spreads over all banks
+    // s ^ (d / 2 % 16)): the lanes of a fragment read spread over 256 bytes
     __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kTileBytes];
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c32 = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -571,9 +577,10 @@ size_t sdpa_mfma_workspace_bytes(int64_t B, int64_t Hq, int64_t Lq, int64_t nspl
 // partials fit max_bytes. On MI355X a 64-key
 // tile of 128 rows took 2.4 us in a block alone on its CU and 3.1 us in each of two
 // that share one, the merge 4 us and its partials (written and read at about 4
-// TB/s). 512 queries of 512 keys stay whole (27 us; in halves 31), 1500 of 4000 too
-// (197; in halves 205), 16 of 4112 take 22 splits (23.5 us; 28.6 with 16 and a merge
-// of one split at a time).
+// TB/s). Forced counts beside the model's: 512 queries of 512 keys whole 30 us (fp32 q,
+// f16 keys; the model's), in halves 34; 1500 of 4000 whole 227 (bf16; the model's), in
+// halves 216, in 16 349; 16 of 4112 whole 159, in halves 86, in 16 28, in 22 (the
+// model's) 26.
 int64_t sdpa_mfma_splits(int64_t B, int64_t Hq, int64_t Hk, int64_t Lq, int64_t Lk, int num_cus, size_t max_bytes) {
     const int64_t blocks = B * Hk * ((Hq / Hk * Lq + kRows - 1) / kRows), tiles = (Lk + kKeys - 1) / kKeys;
     int64_t best = 1;

@@ -396,10 +396,12 @@ __global__ __launch_bounds__(256) void moe_qmv_kernel(MoeArgs a) {
 // 32 rows of a step per stack as 4 loads into LDS of 8 rows each, and a step's
 // weights move from LDS to registers at once, so that the next step's loads are
 // in flight in the same space during its MFMAs; two blocks per CU. At 500 tokens
-// (31 pairs per expert of 2048 x 768) gate + up took 98 us and down 58 us, the
-// dot products 636 and 426; what holds it there is the issue of VALU (the scaling
-// and unpacking, about 44 instructions per 32 x 32 block of 64 k), LDS reads and
-// MFMAs together at two waves per SIMD, not one of them.
+// (31 pairs per expert of 2048 x 768) gate + up take 90 us and down 55 us, the
+// dot products 636 and 426. No unit is near its limit there: of gate + up's time VALU
+// (the scaling and unpacking, about 44 instructions per 32 x 32 block of 64 k) takes
+// 28 %, the MFMA pipes 16 and LDS 9, of down's 36, 14 and 16; the two waves of a SIMD
+// spend 34 and 37 % of their cycles issuing, 36 and 20 ready but behind another
+// instruction, and 30 and 42 waiting (loads, LDS, the two barriers of a step).
 typedef float moe_f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 moe_bf16x8 __attribute__((ext_vector_type(8)));
 
