@@ -501,10 +501,16 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
             if (t >= count) break;
             if constexpr (SPLIT) {
                 const int64_t part = (grow + rr[t]) * a.nsplit + blockIdx.y;
-                *reinterpret_cast<float2*>(a.part_o + part * kDh + 2 * lane) = make_float2(r0[t], r1[t]);
-                // (m, l) in the units of the other rows: no power of two on p here
-                if (lane == 0)
-                    *reinterpret_cast<float2*>(a.part_ml + part * 2) = make_float2(sub[t] * kLog2e + kPShift<F16>, ls[t]);
+                // (m, l) in the units of the other rows, whose sums hold 2^kPShift: into m
+                // over bf16 values, whose sums it could overflow, into the sums over f16
+                // ones (a larger m leaves the merge fewer bits). What rounding m to fp32
+                // takes from it goes into the sums.
+                constexpr float up = F16 ? 0.0f : kPShift<F16>, by = F16 ? 8192.0f : 1.0f;
+                static_assert(!F16 || kPShift<F16> == 13.0f, "2^kPShift");
+                const float ms = sub[t] * kLog2e + up;
+                const float f = by * (sub[t] == ninf ? 1.0f : (float)exp((double)sub[t] - ((double)ms - up) * 0.69314718055994531));
+                *reinterpret_cast<float2*>(a.part_o + part * kDh + 2 * lane) = make_float2(r0[t] * f, r1[t] * f);
+                if (lane == 0) *reinterpret_cast<float2*>(a.part_ml + part * 2) = make_float2(ms, ls[t] * f);
             } else {
                 const int64_t at = row_at(rr[t]) + 2 * lane;
                 store_y(a.out, at, r0[t] / ls[t], a.out_dt);
