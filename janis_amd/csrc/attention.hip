@@ -355,7 +355,8 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
         for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int r = 0; r < 16; r++) o2 = fmaf(o[t][r], o[t][r], o2);
-        bad |= l > 0.0f && pair32<false>(o2) < 0x1p-7f * all;
+        o2 = pair32<false>(o2);  // by every lane
+        bad |= l > 0.0f && o2 < 0x1p-7f * all;
     }
     const uint64_t votes = __ballot(bad && w0 + c32 < n_rows);
     uint32_t again = (uint32_t)votes | (uint32_t)(votes >> 32);  // rows of the wave to compute again
@@ -391,7 +392,7 @@ __global__ __launch_bounds__(256, QN == 3 ? 1 : 2) void sdpa_mfma_kernel(SdpaArg
     // rows of the wave together, so that they share each key's and value's loads (a
     // lane scores a key, and holds two features of the results). q is read from LDS,
     // which the tiles no longer need (the loop's last barrier is behind every wave). A
-    // row whose scores are numbers has its maximum from above, within 2^kLazy; others
+    // row whose scores are numbers takes m (at most kLazy below its maximum); others
     // take a pass over the keys for it. Bound: VALU, about 1800 cycles per row and 64
     // keys. All rows of 32 heads over 8 not finite, 512 of 512 keys: 631 us, 3.2 ms in
     // the per-row kernel; 300 of 300 of one head: 105 us and 141.
